@@ -23,6 +23,10 @@ LIB_DIR = PACKAGE / "_lib"
 LIBRARY = LIB_DIR / "libmdx_hip.so"
 SOURCES = ("graph.hip", "frame.hip", "soap.hip", "soap_mfma.hip", "soap_quad.hip", "soap_block.hip", "neighbor_list.hip",
            "api.hip")
+# the register-coefficient kernel's shapes: one object per l_max and number of
+# radial groups, the slowest to compile first
+SHAPE_SOURCE = "soap_block_shape.hip"
+SHAPES = tuple((l_max, groups) for l_max in range(9, 1, -1) for groups in (3, 2, 1))
 # peak-rate probes for the roofline (bench.py --peaks), a library of their own
 PEAKS_SOURCE = "peaks.hip"
 PEAKS_LIBRARY = LIB_DIR / "libmdx_peaks.so"
@@ -58,23 +62,27 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     OBJ_DIR.mkdir(exist_ok=True)
     LIB_DIR.mkdir(exist_ok=True)
 
-    def compile_one(name: str) -> Path:
-        obj = OBJ_DIR / (Path(name).stem + ".o")
-        cmd = [hipcc, *HIPCC_FLAGS, "-c", str(CSRC / name), "-o", str(obj)]
+    def compile_one(unit: tuple[str, str, tuple[str, ...]]) -> Path:
+        name, stem, defines = unit
+        obj = OBJ_DIR / (stem + ".o")
+        cmd = [hipcc, *HIPCC_FLAGS, *defines, "-c", str(CSRC / name), "-o", str(obj)]
         proc = subprocess.run(cmd, capture_output=True, text=True)
         messages = "\n".join(
             line for line in (proc.stdout + proc.stderr).splitlines()
             if "packed-fp32-ops" not in line
         )
         if proc.returncode != 0:
-            raise RuntimeError(f"hipcc failed for {name}:\n{messages}")
+            raise RuntimeError(f"hipcc failed for {stem}:\n{messages}")
         if verbose and messages.strip():
             print(messages, file=sys.stderr)
         return obj
 
-    workers = jobs or min(len(SOURCES) + 1, int(os.environ.get("MAX_JOBS", "8")))
+    units = [(SHAPE_SOURCE, f"soap_block_{l_max}_{groups}", (f"-DMDX_BLOCK_LM={l_max}", f"-DMDX_BLOCK_KG={groups}"))
+             for l_max, groups in SHAPES]
+    units += [(name, Path(name).stem, ()) for name in (*SOURCES, PEAKS_SOURCE)]
+    workers = jobs or min(len(units), int(os.environ.get("MAX_JOBS", "8")))
     with ThreadPoolExecutor(max_workers=max(1, workers)) as pool:
-        objects = list(pool.map(compile_one, (*SOURCES, PEAKS_SOURCE)))
+        objects = list(pool.map(compile_one, units))
     for library, parts in ((LIBRARY, objects[:-1]), (PEAKS_LIBRARY, objects[-1:])):
         tmp = library.with_suffix(".so.tmp")
         cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-o", str(tmp), *map(str, parts)]

@@ -661,24 +661,16 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
             if (choice == "quad" && plan->quad_waves == 0) {
                 throw mdx::Error(MDX_INVALID_ARGUMENT, "SOAP plan is outside the 4x4-block kernel's limits");
             }
-            // register-coefficient kernel: GTO basis; atom-level rows with
-            // compression off, mu2 or crossover (weighted or not) or mu1nu1
-            // (unweighted), the same rows as float64 partial rows of an outer
-            // average, or inner structure averages without compression
-            // (weighted: large structures only); a compiled (l_max, radial
-            // groups, species) shape.
-            // It keeps its coefficients in registers, so the tile kernel's LDS
-            // limit does not apply to it
-            const int cm = plan->compression;
-            const bool block_rows = (p.average == 0 || p.average == 2) &&
-                                    (cm == 0 || cm == 1 || cm == 3 || (cm == 2 && plan->weighted == 0));
-            const bool block_inner = p.average == 1 && cm == 0;
-            const bool block_options = plan->radial_basis == 0 && (block_rows || block_inner);
-            if (block_options && quad_range && (choice == "auto" || choice == "block")) {
+            // register-coefficient kernel: GTO basis, a compiled (l_max,
+            // radial groups, species) shape.  It keeps its coefficients in
+            // registers, so the tile kernel's LDS limit does not apply to it
+            if (plan->radial_basis == 0 && quad_range && (choice == "auto" || choice == "block")) {
                 mdx::BlockPlanHost bp;
-                // an outer average's rows are float64 partial rows
-                const int row_dtype = p.average == 2 ? 8 : p.out_dtype;
-                if (mdx::block_plan_tables(plan->S, n, p.l_max, row_dtype, cm, beta, pref, expo, bp)) {
+                double beta_largest = 0.0;
+                for (int i = 0; i < L * n * n; ++i) beta_largest = std::max(beta_largest, std::fabs(p.betas[i]));
+                if (mdx::block_plan_tables(plan->S, n, p.l_max, p.out_dtype, p.average, plan->compression,
+                                           plan->weighted != 0, beta_largest, beta, pref, expo, bp)) {
+                    plan->block_table_dtype = bp.table_dtype;
                     plan->block_waves = bp.waves;
                     plan->block_kg = bp.kg;
                     plan->block_ncr = bp.ncr;

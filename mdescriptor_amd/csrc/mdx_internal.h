@@ -472,7 +472,7 @@ struct mdx_soap_plan {
     // register-coefficient kernel (soap_block.hip), default options and
     // average "off" only: wavefronts (0: not used), radial groups,
     // coefficient registers, lane tables
-    int block_waves = 0, block_kg = 0, block_ncr = 0;
+    int block_waves = 0, block_kg = 0, block_ncr = 0, block_table_dtype = 8;
     bool block_forced = false; // MDX_HIP_SOAP_KERNEL=block: also for inner averages of few large structures
     mdx::DeviceBuffer d_block_e1, d_block_beta, d_block_ps;
     // options beyond the GTO / uncompressed / unweighted default (mdx_soap_options)

@@ -398,42 +398,37 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     const int64_t rows = p.average != 0 ? pb.structures : pb.atoms;
     if (rows == 0 || d.F == 0) return;
 
-    // the register-coefficient kernel where the plan chose it (atom-level
-    // rows, with or without weights and with the compressions it takes, or
-    // unweighted, uncompressed structure averages of the inner kind, which it
-    // forms from the structure's centres directly) and every centre's rows
-    // fit their slot codes
-    // It forms a structure's inner average in one workgroup when the
-    // structures are small (a wavefront of atoms) or many enough to fill the
-    // device (four per compute unit); a batch of a few large structures (16
-    // cells of 4,096 atoms: 16 workgroups, 50 ms) sums runs of centres into
-    // partial coefficient rows instead, reduced per structure (1.1 ms).
+    // The register-coefficient kernel where the plan chose it and every
+    // centre's rows fit their slot codes.  It forms a structure's average in
+    // one workgroup when the structures are small (a wavefront of atoms) or
+    // many enough to fill the device (four per compute unit); the inner
+    // averages of a few large structures (16 cells of 4,096 atoms: 16
+    // workgroups, 50 ms) sum runs of centres into partial coefficient rows
+    // instead, reduced per structure (1.1 ms).
     int64_t largest_structure = 0;
     for (size_t st = 0; st + 1 < pb.offsets.size(); ++st) {
         largest_structure = std::max(largest_structure, pb.offsets[st + 1] - pb.offsets[st]);
     }
     const bool inner_fits = largest_structure <= kBlockSmallAtoms || p.block_forced ||
                             pb.structures >= 4 * static_cast<int64_t>(device_compute_units());
-    // Outer averages of the same large structures take it too: every
-    // centre's row as a float64 partial row (at most 4 GiB of them), folded
-    // per structure, then the mean (k_finalize_outer).  Many small
-    // structures keep the 4x4-block kernel, whose partial rows sum runs of
-    // centres in LDS (a row per centre would multiply the traffic by the
-    // run length).
-    const bool outer_fits = (!inner_fits || p.block_forced) && static_cast<double>(pb.atoms) * static_cast<double>(d.F) * 8.0 <= 4294967296.0;
-    // Outer averages of small structures (or of more structures than fill
-    // the device), unweighted and without mu1nu1, take it with a workgroup
-    // per structure: each centre's power spectrum is added into the
-    // structure's float64 row in LDS and the mean written once, with no
-    // partial rows in HBM.
-    const bool outer_lds = p.average == 2 && inner_fits && p.weighted == 0 && p.compression != 2 &&
-                           d.F * static_cast<int64_t>(sizeof(double)) <= kBlockOuterLdsBytes;
-    // (inner averages with neighbour weights only as runs of centres: the
-    // per-structure modes do not weight)
-    const bool block = p.block_waves > 0 &&
-                       (p.average == 0 || (p.average == 2 && (outer_fits || outer_lds)) ||
-                        (p.average == 1 && p.compression == 0 && (p.weighted == 0 || !inner_fits))) &&
-                       g.row_bound < kQuadMaxRows;
+    // Outer averages with a workgroup per structure add each centre's power
+    // spectrum into the structure's float64 row in LDS and write the mean
+    // once, with no partial rows in HBM.  Large structures, and rows past the
+    // LDS, take every centre's row as a float64 partial row (at most 4 GiB of
+    // them), folded per structure, then the mean (k_finalize_outer).
+    const bool outer_lds =
+        p.average == 2 && inner_fits && d.F * static_cast<int64_t>(sizeof(double)) <= kBlockOuterLdsBytes;
+    const bool outer_fits = static_cast<double>(pb.atoms) * static_cast<double>(d.F) * 8.0 <= 4294967296.0;
+    // Three radial groups pad the power spectrum's Gram tiles (a register per
+    // species), which centres of few neighbours do not repay: 1,000 molecules
+    // of 9-29 atoms at n_max 10, l_max 7, 16x16 kernel and here: rows of five
+    // species 835 and 996 us (three: 502 and 425), outer averages of three
+    // 694 and 826, of five 1,325 and 1,439 (rows of condensed cells of five
+    // species 833 and 655)
+    const bool padded = p.block_kg == 3 && p.block_ncr >= (p.average == 2 ? 3 : 5) && p.average != 1 && p.use_mfma &&
+                        !p.block_forced && pb.most_images <= kBlockSmallAtoms;
+    const bool block =
+        p.block_waves > 0 && (p.average != 2 || outer_fits || outer_lds) && !padded && g.row_bound < kQuadMaxRows;
     const bool block_inner = block && p.average == 1 && inner_fits;
     // other inner averages on that kernel: runs of a structure's centres
     // into partial rows, folded, then a launch of one workgroup per structure
@@ -646,32 +641,22 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                 ba.lane_beta = p.d_block_beta.as<double>();
                 ba.ps_offsets = p.d_block_ps.as<int32_t>();
                 ba.S = p.S;
-                ba.out_dtype = block_outer || block_outer_lds ? 8 : p.out_dtype;
+                ba.table_dtype = p.block_table_dtype;
+                ba.out_bytes = block_outer ? 8 : p.out_dtype;
                 ba.F = p.features;
                 ba.item_base = base;
                 ba.items = count;
                 ba.struct_offsets = block_inner || block_outer_lds ? pb.d_offsets.as<int64_t>()
                                     : block_runs                  ? d_item_begin
                                                                   : nullptr;
-                ba.outer_lds = block_outer_lds ? p.out_dtype : 0;
+                ba.outer_lds = block_outer_lds ? 1 : 0;
                 ba.partial_out = block_runs ? d_partial : nullptr;
                 ba.small_structures = block_inner && largest_structure <= kBlockSmallAtoms ? 1 : 0;
                 ba.summed = p.compression == 2 ? 1 : 0;
                 ba.mu2 = p.compression == 1 ? 1 : 0;
-                if (p.weighted != 0) {
-                    ba.weighting = p.weighting;
-                    ba.has_w0 = p.has_w0;
-                    ba.w_r0 = p.w_r0;
-                    ba.w_c = p.w_c;
-                    ba.w_d = p.w_d;
-                    ba.w_m = p.w_m;
-                    ba.w_w0 = p.w_w0;
-                    ba.species_w = p.d_species_w.as<double>();
-                    ba.bin_atom = g.bin_atom.as<int32_t>();
-                    ba.bin_image = g.bin_image.as<int32_t>();
-                    ba.images = pb.d_images.as<ImageDesc>();
-                    ba.row_w = d_row_w;
-                }
+                // without weights every species weight is 1
+                ba.row_w = p.weighted != 0 ? d_row_w : p.d_species_w.as<double>();
+                ba.row_w_mask = p.weighted != 0 ? -1 : 0;
                 ba.out = block_outer ? static_cast<void*>(d_partial) : out_device;
                 ba.pitch = block_outer ? static_cast<int64_t>(partial_width * sizeof(double)) : pitch_bytes;
                 block_args = ba;

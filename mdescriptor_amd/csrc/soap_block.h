@@ -1,26 +1,31 @@
 // Host/device interface of the register-coefficient SOAP kernel
-// (soap_block.hip): GTO basis, no compression; atom-level rows (average
-// "off"), with or without neighbour weights, or a row per structure of its
-// centres' averaged coefficients (average "inner").
+// (soap_block.hip, soap_block_kernel.h): GTO basis, every compression, with
+// or without neighbour weights; a row per centre, or a row per structure of
+// its centres' averaged coefficients (average "inner") or averaged power
+// spectra ("outer").
 #pragma once
 
 #include "mdx_internal.h"
 
 namespace mdx {
 
-// Stream kinds of the kernel: a row per centre; a row per structure (inner
-// average) from a centre-by-centre stream; the same from a species-major
-// stream over the structure's pairs (structures of at most 64 atoms); a row
-// per centre with weighted neighbours; a row per centre of mu1nu1 features
-// (each channel against the species-summed channels); inner averages of
-// large structures in two launches: runs of a structure's centres leave
-// their summed coefficient registers in partial rows (with or without
-// neighbour weights), then a row per structure from the sum of its partial
-// rows; outer averages of structures a workgroup each, every centre's power
-// spectrum added into the structure's float64 row in LDS and the mean
-// written once.
-constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockRowsWeighted = 3, kBlockRowsSummed = 4,
-              kBlockInnerRuns = 5, kBlockInnerFinal = 6, kBlockInnerRunsWeighted = 7, kBlockOuterLds = 8;
+// Kinds of row the kernel is compiled for.
+//   rows         a row per centre
+//   inner        a row per structure of its centres' averaged coefficients,
+//                from a centre-by-centre stream: a workgroup per structure,
+//                or for few large structures two launches (partial_out /
+//                partial_in): runs of a structure's centres leave their
+//                summed coefficient registers in partial rows, then a row per
+//                structure from the sum of its partial rows
+//   inner small  the same from a species-major stream over the structure's
+//                pairs (structures of at most 64 atoms)
+//   outer LDS    outer averages, a workgroup per structure: every centre's
+//                power spectrum added into the structure's float64 row in
+//                LDS and the mean written once
+// Each takes neighbour weights (row_w) and every compression: mu1nu1
+// (summed: each channel against the species-summed channels) as a branch at
+// the end of a row, the others through the plan's tables.
+constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuterLds = 3;
 // largest row (features x 8 bytes) the outer mode accumulates in LDS
 constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;
 constexpr int kBlockSmallAtoms = 64;
@@ -38,7 +43,8 @@ struct BlockArgs {
     const double* lane_beta;    // [l][fold term][64]: beta^T operand of the lane
     const int32_t* ps_offsets;  // [tile pair][value][64]: (byte offset at l = 0) << 9 | feature stride per l
     int S;                      // species
-    int out_dtype;              // 4 or 8 bytes
+    int table_dtype;            // bytes per value the plan's tables are for: 4 (float32 exps and rows) or 8
+    int out_bytes;              // bytes per output value, 4 or 8 (tables for 4: 4)
     int64_t F;                  // features per row
     int64_t item_base, items, per_block; // centres, or structures when struct_offsets is set
     const int64_t* struct_offsets;       // null: a row per centre; else first centre of each structure
@@ -54,8 +60,11 @@ struct BlockArgs {
     const int32_t* bin_image;            // image of each binned image (w0: the exact self pair)
     const int32_t* bin_type;             // species of each binned image
     const ImageDesc* images;             // image table (integer shifts)
-    const double* row_w;                 // weighted modes: each pair row's weight, distance function
-                                         // (or w0) times species weight (k_block_row_weights)
+    // each pair row's weight, at row_w[row & row_w_mask]: the distance
+    // function (or w0) times the species weight (k_block_row_weights), mask
+    // -1; without weights one value of 1, mask 0
+    const double* row_w;
+    int64_t row_w_mask;
     int summed;                          // mu1nu1: spectrum against the species-summed coefficients
     int mu2;                             // mu2: every species' sums into the first species' slots
     // inner averages in two launches: the runs' launch writes partial_out
@@ -68,9 +77,8 @@ struct BlockArgs {
     const double* partial_in;
     const int64_t* part_items;
     // outer averages in LDS (items = structures, struct_offsets = the
-    // batch's atom offsets, out_dtype 8: the plan's tables are those of
-    // float64 rows): a row per structure, the mean of its centres' power
-    // spectra, written with outer_lds bytes per value (4 or 8; 0: off)
+    // batch's atom offsets, table_dtype 8): a row per structure, the mean of
+    // its centres' power spectra
     int outer_lds;
     void* out;
     int64_t pitch;              // bytes between output rows
@@ -83,15 +91,32 @@ struct BlockPlanHost {
     int kg = 0;      // radial groups of 4 channels
     int ncr = 0;     // coefficient registers per (l, column group)
     int waves = 0;   // wavefronts per workgroup
+    int table_dtype = 8;
     std::vector<double> lane_e1, lane_beta;
     std::vector<int32_t> ps_offsets; // packed feature offsets
 };
 
-// Fills out and returns true when (S, n, l_max) is one of the compiled shapes.
+// One compiled shape (soap_block_shape.hip): l_max, radial groups,
+// coefficient registers.  every_form: compiled with float32 and float64 exps
+// for rows and inner averages, weighted or not; else float32 exps serve
+// unweighted rows only, and float64 tables everything else, whatever the
+// output type.
+struct BlockShape {
+    int l_max, kg, ncr;
+    bool every_form;
+    int waves;
+    void (*launch)(hipStream_t, const BlockArgs&, int64_t);
+};
+
+// Fills out and returns true when a compiled shape holds (S, n, l_max).
 // compression: 0 off, 1 mu2 (one coefficient species: the shape of S
 // species, the feature layout of one), 2 mu1nu1, 3 crossover (the feature
-// layouts of soap.cpp:948-1013).
-bool block_plan_tables(int S, int n, int l_max, int out_dtype, int compression, const std::vector<double>& beta_scaled,
+// layouts of soap.cpp:948-1013).  average: 0 off, 1 inner, 2 outer; weighted:
+// neighbour weights.
+// beta_largest is the largest |beta| entry; out.table_dtype the value size
+// the tables are built for.
+bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted,
+                       double beta_largest, const std::vector<double>& beta_scaled,
                        const std::vector<double>& pref, const std::vector<double>& expo, BlockPlanHost& out);
 void launch_block_expand(hipStream_t stream, int l_max, int kg, int ncr, const BlockArgs& a, int64_t count);
 // doubles in one partial row of the runs' launch

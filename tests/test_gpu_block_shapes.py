@@ -1,0 +1,104 @@
+"""The register-coefficient kernel over its compiled shapes, against the oracle.
+
+Every number of radial groups (n_max 1-4, 5-8, 9-12) with every number of
+coefficient registers, exactly filled and rounded up to the next compiled
+one, at the smallest and largest l_max and in between; each average on
+structures of at most a wavefront of atoms and on larger ones; neighbour
+weights and every compression.  Gates as in test_gpu_parity.py: float64
+|delta| <= 1e-10 (|ref| + max|row|), float32 the same form at 2e-5.
+"""
+
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from conftest import scaled_error
+from mdescriptor_amd import _hip
+from mdescriptor_amd.descriptors.basis import basis_gto
+
+pytestmark = pytest.mark.gpu
+
+GATES = {"float64": 1e-10, "float32": 2e-5}
+SPECIES = [1, 6, 7, 8, 9, 14, 15, 16]
+POW_W0 = {"weighting": {"function": "pow", "r0": 2.0, "c": 1.0, "d": 1.0, "m": 4.0, "w0": 0.5}}
+
+# (species, n_max, l_max)
+SHAPES = [
+    (4, 4, 2), (1, 1, 3), (5, 3, 4), (8, 4, 5), (6, 2, 9),            # one radial group
+    (2, 8, 2), (1, 5, 5), (4, 7, 3), (3, 8, 7), (6, 6, 6), (5, 8, 9),  # two
+    (1, 9, 2), (2, 12, 4), (3, 9, 5), (4, 10, 6), (5, 9, 8), (2, 11, 9),  # three (four species: five registers)
+]
+
+
+def _structures(seed, sizes, species):
+    """Alternating periodic boxes and isolated clusters with every species,
+    atoms at least 0.9 A apart."""
+
+    rng = np.random.default_rng(seed)
+    numbers, positions, cells, pbc = [], [], [], []
+    for i, atoms in enumerate(sizes):
+        periodic = i % 2 == 0
+        grid = int(np.ceil(atoms ** (1.0 / 3.0)))
+        sites = np.stack(np.unravel_index(rng.permutation(grid ** 3)[:atoms], (grid,) * 3), axis=1)
+        spacing = 2.2 if periodic else 1.6
+        positions.append((sites + 0.5) * spacing + rng.uniform(-0.3, 0.3, (atoms, 3)))
+        numbers.append(np.resize(species, atoms)[rng.permutation(atoms)])
+        cells.append(np.eye(3) * grid * spacing * (1.0 if periodic else 0.0))
+        pbc.append([1, 1, 1] if periodic else [0, 0, 0])
+    return SimpleNamespace(numbers=np.concatenate(numbers).astype(np.int32), positions=np.concatenate(positions),
+                           cells=np.asarray(cells), pbc=np.asarray(pbc, np.int32),
+                           offsets=np.concatenate([[0], np.cumsum(sizes)]))
+
+
+def _check(ctx, oracle, batch, shape, average, dtype, options=None):
+    count, n_max, l_max = shape
+    species = SPECIES[:count]
+    r_cut = 6.0 if n_max > 8 else 4.0
+    alphas, betas = basis_gto(r_cut, n_max, l_max)
+    arguments = dict(species=species, n_max=n_max, l_max=l_max, r_cut=r_cut, sigma=1.0, alphas=alphas, betas=betas,
+                     average=average, options=options)
+    plan = _hip.SoapPlan(ctx, dtype=dtype, **arguments)
+    try:
+        values, timing = plan.compute(batch)
+    finally:
+        plan.close()
+    assert timing["expansion_tiles"] <= -1000
+    expected = oracle.soap(batch, **arguments)
+    assert values.shape == expected.shape
+    assert np.all(np.isfinite(values))
+    error = scaled_error(values, expected)
+    assert error <= GATES[dtype], f"{shape} {average} {dtype} {options}: scaled error {error:.3e}"
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("average", ["off", "inner", "outer"])
+def test_shape(hip_context, oracle, shape, average):
+    # 21 atoms a structure and a lone atom; then structures past a wavefront,
+    # which an average takes as runs or partial rows
+    for sizes, dtype in (((21, 13, 1, 20), "float64"), ((70, 66), "float32")):
+        _check(hip_context, oracle, _structures(sum(shape), sizes, SPECIES[:shape[0]]), shape, average, dtype)
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 2), (3, 8, 7), (4, 7, 3), (2, 9, 5), (4, 9, 4)])
+@pytest.mark.parametrize("average", ["off", "inner", "outer"])
+@pytest.mark.parametrize("name", ["pow_w0", "species_weights", "mu2", "mu1nu1", "crossover", "pow_w0_mu1nu1"])
+def test_shape_options(hip_context, oracle, shape, average, name):
+    options = {}
+    if "pow_w0" in name:
+        options.update(POW_W0)
+    if name == "species_weights":
+        options["species_weights"] = [0.5 + 0.25 * i for i in range(shape[0])]
+    if name.split("_")[-1] in ("mu2", "mu1nu1", "crossover"):
+        options["compression"] = name.split("_")[-1]
+    for sizes, dtype in (((21, 13, 1, 20), "float64"), ((70, 66), "float32")):
+        _check(hip_context, oracle, _structures(sum(shape), sizes, SPECIES[:shape[0]]), shape, average, dtype, options)
+
+
+def test_outer_average_past_the_lds_row(hip_context, oracle):
+    """Small structures whose row is too wide for the LDS accumulation (more
+    than 48 KB): a float64 partial row per centre."""
+
+    _check(hip_context, oracle, _structures(5, (21, 13, 1, 20), SPECIES[:5]), (5, 9, 8), "outer", "float64")
