@@ -28,8 +28,40 @@
 namespace mdx {
 
 constexpr int kItemCentres = 32;
+constexpr int kFoldItems = 16;  // rows per split, at least
+constexpr int kFoldSplits = 32; // splits per structure, at most
 
 namespace {
+
+// Scratch bytes a run's partial rows may take so that shortening the runs
+// never makes a batch outgrow the no-allocation entry point's static array
+// (whose runs are the same): what the graph leaves of the array, none where
+// that is close, and no such limit where the graph alone is past it.  The
+// graph's share is an estimate from its row slots, bins and cells.
+int64_t partial_budget(const PreparedBatch& pb, const DeviceGraph& g, bool weighted) {
+    const double atoms = static_cast<double>(pb.atoms), S = static_cast<double>(g.n_species);
+    const double rows = atoms * static_cast<double>(g.slots > 0 ? g.slots : g.row_bound);
+    const double graph = rows * (weighted ? 12.0 : 4.0) + atoms * (4.0 * S + 16.0) +
+                         static_cast<double>(pb.ext_total) * 44.0 +
+                         static_cast<double>(pb.cells_total) * (8.0 * S + 48.0);
+    constexpr double kArray = static_cast<double>(MDX_NOALLOC_SCRATCH_BYTES);
+    if (graph > 1.25 * kArray) return int64_t(1) << 30;
+    return std::max<int64_t>(0, static_cast<int64_t>(0.85 * kArray - graph));
+}
+
+// Centres per run of an averaged structure: kItemCentres where the batch then
+// still has a few runs for every compute unit, shorter for smaller batches
+// (8,192 atoms at 32 are 256 runs, one workgroup a compute unit) as far as
+// their partial rows (width doubles each, and the folded ones) fit the budget.
+int64_t run_centres(const PreparedBatch& pb, size_t width, int64_t budget) {
+    const int64_t fill = 8 * static_cast<int64_t>(device_compute_units());
+    int64_t length = std::max<int64_t>(1, std::min<int64_t>(kItemCentres, pb.atoms / fill));
+    auto bytes = [&](int64_t len) {
+        return static_cast<double>(pb.atoms / len + 33 * pb.structures) * static_cast<double>(width) * sizeof(double);
+    };
+    while (length < kItemCentres && bytes(length) > static_cast<double>(budget)) length *= 2;
+    return std::min<int64_t>(length, kItemCentres);
+}
 
 struct SoapDims {
     int S, n, l_max, L, H, LN, CH;
@@ -332,8 +364,6 @@ __global__ __launch_bounds__(kBlock) void k_finalize_outer(const double* partial
 // is zero), and the finalize then walks the structure's splits (at most
 // kFoldSplits).  The order of the sums is fixed, so the result does not
 // depend on the launch.
-constexpr int kFoldItems = 16;  // rows per split, at least
-constexpr int kFoldSplits = 32; // splits per structure, at most
 __global__ __launch_bounds__(kBlock) void k_fold_partials(const double* partial, int64_t width,
                                                           const int64_t* struct_items, int64_t col_tiles,
                                                           int splits, int64_t per_split, double* folded) {
@@ -378,6 +408,116 @@ void dispatch_hpt(int hpt, hipStream_t stream, dim3 grid, size_t lds, const mdx_
     }
 }
 
+// The kernel and the decomposition of a run.
+struct Choice {
+    bool block = false;           // the register-coefficient kernel
+    bool block_inner = false;     // ... a workgroup per structure
+    bool block_runs = false;      // ... runs of a structure's centres into partial coefficient rows
+    bool block_outer = false;     // ... a float64 partial row per centre
+    bool block_outer_lds = false; // ... a workgroup per structure, power spectra summed in LDS
+    bool quad = false;            // the 4x4-block kernel
+    int64_t largest_structure = 0;
+    int64_t run = kItemCentres;   // centres per run
+    size_t partial_width = 0;     // doubles of a partial row
+    bool partials() const { return !block_inner && !block_outer_lds; } // (of an average)
+};
+
+// saving: 0 what is fastest; 1 no more scratch than runs of kItemCentres
+// take; 2 without the register-coefficient kernel's partial rows
+Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g, int64_t budget, int saving) {
+    Choice c;
+    const double F = static_cast<double>(p.features);
+    for (size_t st = 0; st + 1 < pb.offsets.size(); ++st) {
+        c.largest_structure = std::max(c.largest_structure, pb.offsets[st + 1] - pb.offsets[st]);
+    }
+    const int64_t units = device_compute_units();
+    // The register-coefficient kernel where the plan chose it and every
+    // centre's rows fit their slot codes.  It forms a structure's average in
+    // one workgroup when the structures are small (a wavefront of atoms) or
+    // many enough to fill the device (four per compute unit); the inner
+    // averages of a few large structures (16 cells of 4,096 atoms: 16
+    // workgroups, 50 ms) sum runs of centres into partial coefficient rows
+    // instead, reduced per structure (1.1 ms).
+    const bool whole = c.largest_structure <= kBlockSmallAtoms || p.block_forced || pb.structures >= 4 * units;
+    // Outer averages with a workgroup per structure add each centre's power
+    // spectrum into the structure's float64 row in LDS and write the mean
+    // once, with no partial rows in HBM.  Large structures, and rows past the
+    // LDS, take every centre's row as a float64 partial row (at most 4 GiB of
+    // them), folded per structure, then the mean (k_finalize_outer); so do
+    // fewer structures than two per compute unit, which spread over the
+    // device better, where the scratch allows.
+    const double centre_rows = static_cast<double>(pb.atoms + 5 * pb.structures) * F * 8.0;
+    const bool few = pb.structures < 2 * units && centre_rows <= static_cast<double>(budget);
+    const bool outer_lds = p.average == 2 && whole && F * sizeof(double) <= static_cast<double>(kBlockOuterLdsBytes) &&
+                           (!few || saving > 0);
+    const bool outer_rows = static_cast<double>(pb.atoms) * F * 8.0 <= 4294967296.0;
+    // Three radial groups pad the power spectrum's Gram tiles (a register per
+    // species), which centres of few neighbours do not repay: 1,000 molecules
+    // of 9-29 atoms at n_max 10, l_max 7, 16x16 kernel and here: rows of five
+    // species 835 and 996 us (three: 502 and 425), outer averages of three
+    // 694 and 826, of five 1,325 and 1,439 (rows of condensed cells of five
+    // species 833 and 655)
+    const bool padded = p.block_kg == 3 && p.block_ncr >= (p.average == 2 ? 3 : 5) && p.average != 1 && p.use_mfma &&
+                        !p.block_forced && pb.most_images <= kBlockSmallAtoms;
+    c.block = p.block_waves > 0 && (p.average != 2 || outer_rows || outer_lds) && !padded && g.row_bound < kQuadMaxRows;
+    const size_t block_width = c.block ? static_cast<size_t>(block_partial_width(p.l_max, p.block_ncr)) : 0;
+    // A few small periodic structures hold thousands of pairs each (a
+    // workgroup takes about a microsecond per 32 of them): runs too.
+    const bool spread = saving == 0 && !p.block_forced && pb.structures < units &&
+                        c.largest_structure * std::min(pb.most_images, g.row_bound) > kBlockSpreadPairs &&
+                        static_cast<double>(pb.atoms + 5 * pb.structures) * static_cast<double>(block_width) * 8.0 <=
+                            static_cast<double>(budget);
+    c.block_inner = c.block && p.average == 1 && whole && !spread;
+    c.block_outer_lds = c.block && outer_lds;
+    c.block_runs = c.block && p.average == 1 && !c.block_inner;
+    c.block_outer = c.block && p.average == 2 && !outer_lds;
+    if (saving == 2 && (c.block_runs || c.block_outer) && !p.block_forced) {
+        c.block = c.block_runs = c.block_outer = false;
+    }
+    // else the 4x4-block kernel where the plan chose it (its coefficient rows
+    // are its own), the 16x16 kernel, the generic one
+    c.quad = !c.block && p.use_mfma && p.quad_waves > 0 && g.row_bound < kQuadMaxRows;
+    const int rows = c.quad ? quad_coefficient_rows(p.Sc, p.n) : mfma_coefficient_rows(p.Sc, p.n, p.compression);
+    c.partial_width = c.block_runs     ? block_width
+                      : p.average != 1 ? static_cast<size_t>(p.features)
+                      : p.use_mfma     ? static_cast<size_t>(rows) * static_cast<size_t>(p.hpad)
+                                       : static_cast<size_t>(p.coeff_size);
+    if (p.average != 0 && c.partials() && !c.block_outer) {
+        c.run = saving == 0 ? run_centres(pb, c.partial_width, budget) : kItemCentres;
+    }
+    return c;
+}
+
+// Bytes of the folded rows' splits: see k_fold_partials.
+struct Fold {
+    int splits = 0;
+    int64_t per_split = 0;
+};
+Fold fold_of(int64_t most_items) {
+    Fold f;
+    if (most_items > 2 * kFoldItems) {
+        f.splits = static_cast<int>(std::min<int64_t>((most_items + kFoldItems - 1) / kFoldItems, kFoldSplits));
+        f.per_split = (most_items + f.splits - 1) / f.splits;
+    }
+    return f;
+}
+
+// Scratch of a run: its partial rows, folded rows, item tables and row weights.
+size_t scratch_bytes(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g, const Choice& c) {
+    size_t bytes = c.block && p.weighted != 0 ? (g.pair_bin.bytes / sizeof(uint32_t)) * sizeof(double) + 256 : 0;
+    if (p.average == 0 || !c.partials()) return bytes;
+    const int64_t run = c.block_outer ? 1 : c.run;
+    int64_t items = 0, most = 0;
+    for (size_t st = 0; st + 1 < pb.offsets.size(); ++st) {
+        const int64_t n = (pb.offsets[st + 1] - pb.offsets[st] + run - 1) / run;
+        items += n;
+        most = std::max(most, n);
+    }
+    const size_t folded = static_cast<size_t>(pb.structures) * static_cast<size_t>(fold_of(most).splits);
+    return bytes + (static_cast<size_t>(items) + folded) * c.partial_width * sizeof(double) +
+           (static_cast<size_t>(items) + 2 * static_cast<size_t>(pb.structures) + 4) * sizeof(int64_t) + 1024;
+}
+
 } // namespace
 
 void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, const DeviceGraph& g,
@@ -398,43 +538,19 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     const int64_t rows = p.average != 0 ? pb.structures : pb.atoms;
     if (rows == 0 || d.F == 0) return;
 
-    // The register-coefficient kernel where the plan chose it and every
-    // centre's rows fit their slot codes.  It forms a structure's average in
-    // one workgroup when the structures are small (a wavefront of atoms) or
-    // many enough to fill the device (four per compute unit); the inner
-    // averages of a few large structures (16 cells of 4,096 atoms: 16
-    // workgroups, 50 ms) sum runs of centres into partial coefficient rows
-    // instead, reduced per structure (1.1 ms).
-    int64_t largest_structure = 0;
-    for (size_t st = 0; st + 1 < pb.offsets.size(); ++st) {
-        largest_structure = std::max(largest_structure, pb.offsets[st + 1] - pb.offsets[st]);
+    const int64_t budget = partial_budget(pb, g, p.weighted != 0);
+    Choice choice = choose(p, pb, g, budget, 0);
+    if (partials.arena != nullptr) {
+        // the static array of a no-allocation run: what does not fit there
+        // takes long runs, then the tile kernels' short partial rows
+        for (int saving = 1; saving <= 2 && scratch_bytes(p, pb, g, choice) > partials.arena->left() + partials.bytes; ++saving) {
+            choice = choose(p, pb, g, budget, saving);
+        }
     }
-    const bool inner_fits = largest_structure <= kBlockSmallAtoms || p.block_forced ||
-                            pb.structures >= 4 * static_cast<int64_t>(device_compute_units());
-    // Outer averages with a workgroup per structure add each centre's power
-    // spectrum into the structure's float64 row in LDS and write the mean
-    // once, with no partial rows in HBM.  Large structures, and rows past the
-    // LDS, take every centre's row as a float64 partial row (at most 4 GiB of
-    // them), folded per structure, then the mean (k_finalize_outer).
-    const bool outer_lds =
-        p.average == 2 && inner_fits && d.F * static_cast<int64_t>(sizeof(double)) <= kBlockOuterLdsBytes;
-    const bool outer_fits = static_cast<double>(pb.atoms) * static_cast<double>(d.F) * 8.0 <= 4294967296.0;
-    // Three radial groups pad the power spectrum's Gram tiles (a register per
-    // species), which centres of few neighbours do not repay: 1,000 molecules
-    // of 9-29 atoms at n_max 10, l_max 7, 16x16 kernel and here: rows of five
-    // species 835 and 996 us (three: 502 and 425), outer averages of three
-    // 694 and 826, of five 1,325 and 1,439 (rows of condensed cells of five
-    // species 833 and 655)
-    const bool padded = p.block_kg == 3 && p.block_ncr >= (p.average == 2 ? 3 : 5) && p.average != 1 && p.use_mfma &&
-                        !p.block_forced && pb.most_images <= kBlockSmallAtoms;
-    const bool block =
-        p.block_waves > 0 && (p.average != 2 || outer_fits || outer_lds) && !padded && g.row_bound < kQuadMaxRows;
-    const bool block_inner = block && p.average == 1 && inner_fits;
-    // other inner averages on that kernel: runs of a structure's centres
-    // into partial rows, folded, then a launch of one workgroup per structure
-    const bool block_runs = block && p.average == 1 && !inner_fits;
-    const bool block_outer_lds = block && outer_lds;
-    const bool block_outer = block && p.average == 2 && !outer_lds;
+    const bool block = choice.block, block_inner = choice.block_inner, block_runs = choice.block_runs;
+    const bool block_outer = choice.block_outer, block_outer_lds = choice.block_outer_lds;
+    const int64_t largest_structure = choice.largest_structure;
+    const size_t partial_width = choice.partial_width;
 
     // work items
     std::vector<int64_t>& item_begin_h = pb.item_begin;
@@ -450,7 +566,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         for (int64_t s = 0; s < pb.structures; ++s) {
             struct_items_h[static_cast<size_t>(s)] = static_cast<int64_t>(item_begin_h.size());
             for (int64_t a = pb.offsets[static_cast<size_t>(s)]; a < pb.offsets[static_cast<size_t>(s) + 1];
-                 a += kItemCentres) {
+                 a += choice.run) {
                 item_begin_h.push_back(a);
             }
         }
@@ -466,7 +582,6 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     // folded rows and their structure ranges
     int fold_splits = 0;
     int64_t fold_per_split = 0;
-    size_t partial_width = 0;
     double* d_folded = nullptr;
     // weighted plans on the register-coefficient kernel: each pair row's
     // weight, computed once before the expansion (k_block_row_weights), after
@@ -477,20 +592,14 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     int64_t* d_fold_items = nullptr;
     std::vector<int64_t>& fold_items_h = pb.fold_items;
     if (p.average != 0 && !block_inner && !block_outer_lds) {
-        const size_t inner_width = p.use_mfma ? static_cast<size_t>(mfma_coefficient_rows(p.Sc, p.n, p.compression)) * static_cast<size_t>(p.hpad)
-                                              : static_cast<size_t>(d.C);
-        const size_t width = block_runs ? static_cast<size_t>(block_partial_width(p.l_max, p.block_ncr))
-                             : p.average == 1 ? inner_width
-                                              : static_cast<size_t>(d.F);
-        partial_width = width;
+        const size_t width = partial_width;
         int64_t most_items = 0;
         for (int64_t s = 0; s < pb.structures; ++s) {
             most_items = std::max(most_items, struct_items_h[static_cast<size_t>(s) + 1] - struct_items_h[static_cast<size_t>(s)]);
         }
-        if (most_items > 2 * kFoldItems) {
-            fold_splits = static_cast<int>(std::min<int64_t>((most_items + kFoldItems - 1) / kFoldItems, kFoldSplits));
-            fold_per_split = (most_items + fold_splits - 1) / fold_splits;
-        }
+        const Fold f = fold_of(most_items);
+        fold_splits = f.splits;
+        fold_per_split = f.per_split;
         fold_items_h.clear();
         if (fold_splits > 0) {
             for (int64_t s = 0; s <= pb.structures; ++s) fold_items_h.push_back(s * fold_splits);
@@ -544,8 +653,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     const bool hook = on_slice != nullptr && *on_slice && p.average == 0;
     int64_t launches = 0;
     if (block || p.use_mfma) {
-        // else the 4x4-block kernel where the plan chose it
-        const bool quad = !block && p.quad_waves > 0 && g.row_bound < kQuadMaxRows;
+        const bool quad = choice.quad;
         MfmaDims md{};
         md.S = p.S;
         md.n = p.n;
@@ -716,9 +824,9 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     }
     const int64_t acc_words = p.average == 1 ? d.C : p.average == 2 ? d.F : 0;
     // chunk of neighbours staged per step: largest that keeps LDS within budget
-    const size_t budget = 64 * 1024;
+    const size_t lds_budget = 64 * 1024;
     int CH = 64;
-    while (CH > 8 && expand_lds_bytes(p, CH, 0) > budget) CH /= 2;
+    while (CH > 8 && expand_lds_bytes(p, CH, 0) > lds_budget) CH /= 2;
     d.CH = CH;
     d.acc_in_lds = acc_words > 0 && expand_lds_bytes(p, CH, static_cast<int>(acc_words)) <= 96 * 1024 ? 1 : 0;
     const size_t lds = expand_lds_bytes(p, CH, d.acc_in_lds ? static_cast<int>(acc_words) : 0);

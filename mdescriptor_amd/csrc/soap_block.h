@@ -29,6 +29,9 @@ constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuter
 // largest row (features x 8 bytes) the outer mode accumulates in LDS
 constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;
 constexpr int kBlockSmallAtoms = 64;
+// pairs of a structure past which a batch of fewer structures than compute
+// units sums runs of its centres instead of whole structures
+constexpr int64_t kBlockSpreadPairs = 4096;
 
 // Launch arguments (one struct, passed by value).
 struct BlockArgs {
