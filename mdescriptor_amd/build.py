@@ -21,8 +21,8 @@ CSRC = PACKAGE / "csrc"
 OBJ_DIR = PACKAGE / "_build"
 LIB_DIR = PACKAGE / "_lib"
 LIBRARY = LIB_DIR / "libmdx_hip.so"
-SOURCES = ("graph.hip", "frame.hip", "soap.hip", "soap_mfma.hip", "soap_quad.hip", "soap_block.hip", "neighbor_list.hip",
-           "api.hip")
+SOURCES = ("graph.hip", "frame.hip", "soap.hip", "soap_mfma.hip", "soap_quad.hip", "soap_block.hip", "soap_poly.hip",
+           "neighbor_list.hip", "api.hip")
 # the register-coefficient kernel's shapes: one object per l_max and number of
 # radial groups, the slowest to compile first
 SHAPE_SOURCE = "soap_block_shape.hip"

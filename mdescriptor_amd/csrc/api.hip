@@ -564,7 +564,7 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
                 // quadrature-weighted basis values w_q r_q^2 g_k(r_q), [q * n + k] (soap.cpp:551-565)
                 const int Q = o->grid_size;
                 plan->grid_size = Q;
-                std::vector<double> bw(static_cast<size_t>(Q) * n), grid(o->radial_grid, o->radial_grid + Q);
+                std::vector<double> bw(static_cast<size_t>(Q) * n);
                 for (int q = 0; q < Q; ++q) {
                     const double radial = o->radial_grid[q];
                     const double quadrature = o->radial_weights[q] * radial * radial;
@@ -572,8 +572,7 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
                         bw[static_cast<size_t>(q) * n + k] = quadrature * o->radial_values[static_cast<size_t>(k) * Q + q];
                     }
                 }
-                upload(plan->d_poly_bw, bw);
-                upload(plan->d_poly_grid, grid);
+                upload(plan->d_poly, mdx::poly_radial_tables(Q, n, eta, o->radial_grid, bw));
             }
             std::vector<double> ps_pref(static_cast<size_t>(L));
             for (int l = 0; l < L; ++l) ps_pref[static_cast<size_t>(l)] = pi * std::sqrt(8.0 / (2.0 * l + 1.0));
@@ -635,7 +634,7 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
             plan->clamp = md.clamp;
             // the workgroup's LDS: 160 KiB on gfx950 (dynamic, no opt-in needed)
             const size_t lds_limit = mdx::device_workgroup_lds();
-            const bool fits = mdx::mfma_template_tiles(mp.tiles) > 0 && mdx::mfma_lds_bytes(md) <= lds_limit;
+            const bool fits = mdx::mfma_template_tiles(mp.tiles) > 0 && mdx::mfma_lds_bytes(md) + mdx::mfma_plan_reserve(md) <= lds_limit;
             // only the matrix-core kernel implements weighting, compression and the polynomial basis
             const bool defaults = plan->compression == 0 && plan->radial_basis == 0 && plan->weighted == 0;
             plan->use_mfma = fits && (choice != "generic" || !defaults);
@@ -661,15 +660,15 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
             if (choice == "quad" && plan->quad_waves == 0) {
                 throw mdx::Error(MDX_INVALID_ARGUMENT, "SOAP plan is outside the 4x4-block kernel's limits");
             }
-            // register-coefficient kernel: GTO basis, a compiled (l_max,
-            // radial groups, species) shape.  It keeps its coefficients in
-            // registers, so the tile kernel's LDS limit does not apply to it
-            if (plan->radial_basis == 0 && quad_range && (choice == "auto" || choice == "block")) {
+            // register-coefficient kernel: a compiled (l_max, radial groups,
+            // species) shape.  It keeps its coefficients in registers, so the
+            // tile kernel's LDS limit does not apply to it
+            if (quad_range && (choice == "auto" || choice == "block")) {
                 mdx::BlockPlanHost bp;
                 double beta_largest = 0.0;
-                for (int i = 0; i < L * n * n; ++i) beta_largest = std::max(beta_largest, std::fabs(p.betas[i]));
+                for (int i = 0; plan->radial_basis == 0 && i < L * n * n; ++i) beta_largest = std::max(beta_largest, std::fabs(p.betas[i]));
                 if (mdx::block_plan_tables(plan->S, n, p.l_max, p.out_dtype, p.average, plan->compression,
-                                           plan->weighted != 0, beta_largest, beta, pref, expo, bp)) {
+                                           plan->weighted != 0, plan->radial_basis == 1, beta_largest, beta, pref, expo, bp)) {
                     plan->block_table_dtype = bp.table_dtype;
                     plan->block_waves = bp.waves;
                     plan->block_kg = bp.kg;

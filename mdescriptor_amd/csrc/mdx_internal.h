@@ -485,7 +485,7 @@ struct mdx_soap_plan {
     int weighted = 0;        // any weighting function, w0 or species weight != 1
     double w_r0 = 1.0, w_c = 1.0, w_d = 0.0, w_m = 1.0, w_w0 = 1.0, eta = 0.5;
     std::vector<double> species_weights;
-    mdx::DeviceBuffer d_species_w, d_poly_bw, d_poly_grid;
+    mdx::DeviceBuffer d_species_w, d_poly;
 };
 
 struct mdx_device_batch {

@@ -28,6 +28,9 @@
 namespace mdx {
 
 constexpr int kItemCentres = 32;
+// polynomial basis: bytes of radial functions a slice of centres holds, at
+// most (what the last-level cache keeps between the two kernels of a slice)
+constexpr int64_t kPolySliceBytes = int64_t(256) << 20;
 constexpr int kFoldItems = 16;  // rows per split, at least
 constexpr int kFoldSplits = 32; // splits per structure, at most
 
@@ -448,7 +451,7 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
     // device better, where the scratch allows.
     const double centre_rows = static_cast<double>(pb.atoms + 5 * pb.structures) * F * 8.0;
     const bool few = pb.structures < 2 * units && centre_rows <= static_cast<double>(budget);
-    const bool outer_lds = p.average == 2 && whole && F * sizeof(double) <= static_cast<double>(kBlockOuterLdsBytes) &&
+    const bool outer_lds = p.average == 2 && whole && p.radial_basis == 0 && F * sizeof(double) <= static_cast<double>(kBlockOuterLdsBytes) &&
                            (!few || saving > 0);
     const bool outer_rows = static_cast<double>(pb.atoms) * F * 8.0 <= 4294967296.0;
     // Three radial groups pad the power spectrum's Gram tiles (a register per
@@ -589,6 +592,34 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     const size_t row_w_bytes =
         block && p.weighted != 0 ? ((g.pair_bin.bytes / sizeof(uint32_t)) * sizeof(double) + 255) & ~size_t(255) : 0;
     double* d_row_w = nullptr;
+    // polynomial basis: the radial functions of a slice of centres, beside
+    // any partial rows and row weights
+    auto first_centre = [&](int64_t item) {
+        return block_inner ? pb.offsets[static_cast<size_t>(item)]
+               : item_begin_h.empty() ? item
+                                      : item_begin_h[static_cast<size_t>(item)];
+    };
+    int64_t poly_centres = 0, step_groups = 0;
+    size_t poly_bytes = 0;
+    if (p.radial_basis == 1) {
+        const int64_t rows = std::max<int64_t>(1, g.row_bound);
+        int64_t centre_bytes = rows * p.L * p.n * static_cast<int64_t>(sizeof(double));
+        if (block) {
+            // every species' rows padded to whole step groups
+            const int64_t slots = p.block_kg == 2 ? 8 : 16;
+            step_groups = rows / slots + p.S;
+            centre_bytes = step_groups * p.L * kWave * static_cast<int64_t>(sizeof(double));
+        }
+        int64_t room = kPolySliceBytes;
+        if (partials.arena != nullptr) {
+            const size_t left = partials.arena->left() + partials.bytes, used = scratch_bytes(p, pb, g, choice) + 4096;
+            room = std::min(room, static_cast<int64_t>(left > used ? left - used : 0));
+        }
+        poly_centres = room / centre_bytes;
+        for (int64_t it = 0; it < items; ++it) poly_centres = std::max(poly_centres, first_centre(it + 1) - first_centre(it));
+        poly_bytes = (static_cast<size_t>(std::min(poly_centres, pb.atoms) * centre_bytes) + 255) & ~size_t(255);
+    }
+    double* d_poly = nullptr;
     int64_t* d_fold_items = nullptr;
     std::vector<int64_t>& fold_items_h = pb.fold_items;
     if (p.average != 0 && !block_inner && !block_outer_lds) {
@@ -610,7 +641,11 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         const size_t folded_bytes =
             (static_cast<size_t>(pb.structures) * static_cast<size_t>(fold_splits) * width * sizeof(double) + 255) &
             ~size_t(255);
-        scratch.reserve(head + partial_bytes + folded_bytes + row_w_bytes);
+        scratch.reserve(head + partial_bytes + folded_bytes + row_w_bytes + poly_bytes);
+        if (poly_bytes > 0) {
+            d_poly = reinterpret_cast<double*>(static_cast<char*>(scratch.ptr) + head + partial_bytes + folded_bytes +
+                                               row_w_bytes);
+        }
         if (row_w_bytes > 0) {
             d_row_w = reinterpret_cast<double*>(static_cast<char*>(scratch.ptr) + head + partial_bytes + folded_bytes);
         }
@@ -630,9 +665,10 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                                    hipMemcpyHostToDevice, stream));
         }
     }
-    if (row_w_bytes > 0 && d_row_w == nullptr) {
-        scratch.reserve(row_w_bytes);
-        d_row_w = scratch.as<double>();
+    if (row_w_bytes + poly_bytes > 0 && d_row_w == nullptr && d_poly == nullptr) {
+        scratch.reserve(row_w_bytes + poly_bytes);
+        if (row_w_bytes > 0) d_row_w = scratch.as<double>();
+        if (poly_bytes > 0) d_poly = reinterpret_cast<double*>(static_cast<char*>(scratch.ptr) + row_w_bytes);
     }
     // the partial rows the finalize kernels walk, folded first where
     // structures have many items
@@ -691,8 +727,8 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         tab.fbase = p.d_fbase.as<int32_t>();
         tab.fstride = p.d_fstride.as<int32_t>();
         tab.species_w = p.d_species_w.as<double>();
-        tab.poly_bw = p.d_poly_bw.as<double>();
-        tab.poly_grid = p.d_poly_grid.as<double>();
+        tab.poly_g = d_poly;
+        tab.poly_start = g.pair_start.as<int64_t>();
         tab.bin_atom = g.bin_atom.as<int32_t>();
         tab.bin_image = g.bin_image.as<int32_t>();
         tab.images = pb.d_images.as<ImageDesc>();
@@ -733,9 +769,18 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
             }
         }
         if (events != nullptr) MDX_HIP(hipEventRecord(events[2], stream));
-        for (int64_t base = 0; base < items; base += slice) {
+        int64_t count = 0;
+        for (int64_t base = 0; base < items; base += count) {
             if (cancel != nullptr && *cancel != 0) throw Error(MDX_CANCELLED, "descriptor computation was cancelled");
-            const int64_t count = std::min(slice, items - base);
+            count = std::min(slice, items - base);
+            if (p.radial_basis == 1) {
+                // as many items as the radial functions have room for
+                const int64_t first = first_centre(base), most = count;
+                for (count = 1; count < most && first_centre(base + count + 1) - first <= poly_centres;) ++count;
+                md.poly_first = first;
+                launch_poly_radial(stream, pb, g, p.d_poly.as<double>(), md, first, first_centre(base + count) - first,
+                                   step_groups, d_poly);
+            }
             if (block) {
                 BlockArgs ba{};
                 ba.positions = pb.d_positions.as<double>();
@@ -759,12 +804,16 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                                                                   : nullptr;
                 ba.outer_lds = block_outer_lds ? 1 : 0;
                 ba.partial_out = block_runs ? d_partial : nullptr;
-                ba.small_structures = block_inner && largest_structure <= kBlockSmallAtoms ? 1 : 0;
+                ba.small_structures =
+                    block_inner && largest_structure <= kBlockSmallAtoms && p.radial_basis == 0 ? 1 : 0;
                 ba.summed = p.compression == 2 ? 1 : 0;
                 ba.mu2 = p.compression == 1 ? 1 : 0;
                 // without weights every species weight is 1
                 ba.row_w = p.weighted != 0 ? d_row_w : p.d_species_w.as<double>();
                 ba.row_w_mask = p.weighted != 0 ? -1 : 0;
+                ba.poly_g = d_poly;
+                ba.poly_first = md.poly_first;
+                ba.poly_groups = step_groups;
                 ba.out = block_outer ? static_cast<void*>(d_partial) : out_device;
                 ba.pitch = block_outer ? static_cast<int64_t>(partial_width * sizeof(double)) : pitch_bytes;
                 block_args = ba;

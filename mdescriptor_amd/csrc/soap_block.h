@@ -26,6 +26,12 @@ namespace mdx {
 // (summed: each channel against the species-summed channels) as a branch at
 // the end of a row, the others through the plan's tables.
 constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuterLds = 3;
+// ... and forms: unweighted, weighted (the weights may be 1), and the
+// polynomial basis (weighted the same way): the radial functions come from
+// memory (launch_poly_radial) instead of exps, rows and inner averages only,
+// up to two radial groups (its normalisation fails past eight channels).
+constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2;
+constexpr int kBlockPolyGroups = 2;
 // largest row (features x 8 bytes) the outer mode accumulates in LDS
 constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;
 constexpr int kBlockSmallAtoms = 64;
@@ -68,6 +74,11 @@ struct BlockArgs {
     // -1; without weights one value of 1, mask 0
     const double* row_w;
     int64_t row_w_mask;
+    // polynomial basis: radial functions of the slice's pairs, a step group
+    // of 64 values per degree and exp register at
+    // [(centre - poly_first) * poly_groups + group][l][register][lane]
+    const double* poly_g;
+    int64_t poly_first, poly_groups;
     int summed;                          // mu1nu1: spectrum against the species-summed coefficients
     int mu2;                             // mu2: every species' sums into the first species' slots
     // inner averages in two launches: the runs' launch writes partial_out
@@ -115,10 +126,10 @@ struct BlockShape {
 // compression: 0 off, 1 mu2 (one coefficient species: the shape of S
 // species, the feature layout of one), 2 mu1nu1, 3 crossover (the feature
 // layouts of soap.cpp:948-1013).  average: 0 off, 1 inner, 2 outer; weighted:
-// neighbour weights.
+// neighbour weights; polynomial: that radial basis (float64 tables).
 // beta_largest is the largest |beta| entry; out.table_dtype the value size
 // the tables are built for.
-bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted,
+bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted, bool polynomial,
                        double beta_largest, const std::vector<double>& beta_scaled,
                        const std::vector<double>& pref, const std::vector<double>& expo, BlockPlanHost& out);
 void launch_block_expand(hipStream_t stream, int l_max, int kg, int ncr, const BlockArgs& a, int64_t count);

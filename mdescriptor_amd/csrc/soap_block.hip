@@ -44,7 +44,7 @@ int64_t block_partial_width(int l_max, int ncr) {
     return static_cast<int64_t>(units_total(0xffffffffu, l_max + 1)) * ncr * kWaveThreads;
 }
 
-bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted,
+bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted, bool polynomial,
                        double beta_largest, const std::vector<double>& beta_scaled,
                        const std::vector<double>& pref, const std::vector<double>& expo, BlockPlanHost& out) {
     out = BlockPlanHost{};
@@ -52,7 +52,7 @@ bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int 
     // species of the coefficients and the feature layout (mu2: one)
     const int St = compression == 1 ? 1 : S;
     const int kg = (n + 3) / 4;
-    if (n < 1 || kg > 3) return false;
+    if (n < 1 || kg > (polynomial ? kBlockPolyGroups : 3)) return false;
     const BlockShape* e = find_shape(l_max, kg, coefficient_registers(St, kg));
     if (e == nullptr) return false;
     // registers past the species' stay zero, and no feature is stored from them
@@ -63,7 +63,7 @@ bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int 
     // 1.3e4), or the shapes measured with it (twelve channels in 5.5 A, 1.2e5:
     // rows 2.7e-8 off the exact values against 2.5e-8 of rounding)
     const bool f32_exps =
-        e->every_form ? average != 2 : average == 0 && !weighted && beta_largest <= kFloat32ExpBeta;
+        !polynomial && e->every_form ? average != 2 : !polynomial && average == 0 && !weighted && beta_largest <= kFloat32ExpBeta;
     const int table_dtype = f32_exps ? out_dtype : 8;
     out.table_dtype = table_dtype;
     const int L = l_max + 1;
@@ -209,7 +209,8 @@ void launch_block_expand(hipStream_t stream, int l_max, int kg, int ncr, const B
                              a.F * static_cast<int64_t>(sizeof(double)) > kBlockOuterLdsBytes)) {
         throw Error(MDX_INTERNAL, "outer average row does not fit the register-coefficient kernel's LDS");
     }
-    if (a.out_bytes > a.table_dtype || a.row_w == nullptr) {
+    if (a.out_bytes > a.table_dtype || a.row_w == nullptr ||
+        (a.poly_g != nullptr && (kg > kBlockPolyGroups || a.table_dtype != 8 || a.small_structures || a.outer_lds != 0))) {
         throw Error(MDX_INTERNAL, "register-coefficient kernel launched with inconsistent arguments");
     }
     e->launch(stream, a, count);

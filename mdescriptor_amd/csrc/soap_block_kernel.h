@@ -374,7 +374,7 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
     return static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo));
 }
 
-template <int LM, int KG, int NCR, int ES, int MODE, bool kWeighted, int W>
+template <int LM, int KG, int NCR, int ES, int MODE, int FORM, int W>
 __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, const int* s_ps, double* s_acc) {
     using PL = BlockPlan<LM, KG>;
     constexpr int L = PL::L, R = PL::R, P = PL::P, RPL = PL::RPL, NT = PL::NT, GS = PL::GS;
@@ -435,6 +435,8 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     // rows of structure averages (the runs' launch sums a run of a structure's
     // centres the same way, into a partial row)
     constexpr bool inner = MODE != kBlockRows;
+    constexpr bool kPoly = FORM == kBlockPolynomial;
+    constexpr bool kWeighted = FORM != kBlockPlain;
     // outer averages in LDS: a structure's centres one by one, each centre's
     // power spectrum added into s_acc (F float64 values), its mean written
     // when the structure ends
@@ -473,6 +475,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     int64_t st_row = 0;                // pair row of the next chunk's first slot
     int st_q = 0;                      // species of the next chunk
     int st_left = 0;                   // rows of species st_q not yet in a chunk
+    int64_t st_group = 0;              // polynomial basis: the next chunk's first step group
     uint32_t st_more = 0;              // species after st_q with rows (bit mask)
     auto next_species = [&]() {
         st_q = __builtin_amdgcn_readfirstlane(__builtin_ctz(st_more));
@@ -490,6 +493,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
         }
         cnt = pre_count;
         st_row = uniform64(pre_start);
+        if constexpr (kPoly) st_group = (st_centre - a.poly_first) * a.poly_groups;
         st_more = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(__ballot(lane < S && cnt > 0)));
         cnt = lane < S ? cnt : 0;
         prefetch_centre(st_centre + 1);
@@ -558,9 +562,10 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
         int64_t row;    // output row (centre, or structure)
         int catom;      // species-major: centre (atom) of the lane's slot
         double w;       // kWeighted: weight of the lane's slot row (1 without weights)
+        int64_t group;  // polynomial basis: first step group in the radial functions
     };
     auto next_stage = [&]() -> Stage {
-        Stage s{-1, 0, 0, 0, false, false, 0u, 0, 0, 0.0};
+        Stage s{-1, 0, 0, 0, false, false, 0u, 0, 0, 0.0, 0};
         if constexpr (kSpeciesMajor) {
             if (sm_base >= sm_total) {
                 if (st_more == 0) {
@@ -626,6 +631,10 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
             const int64_t slot_row = n > 0 ? st_row + min(lane / 2, n - 1) : 0;
             s.bin = a.pair_bin[slot_row];
             if constexpr (kWeighted) s.w = a.row_w[slot_row & a.row_w_mask];
+        }
+        if constexpr (kPoly) {
+            s.group = st_group;
+            st_group = uniform64(st_group + s.groups);
         }
         st_row = uniform64(st_row + n);
         st_left = __builtin_amdgcn_readfirstlane(st_left - n);
@@ -860,9 +869,9 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     };
     // harmonics of a stage's slots from the centre position (cx, cy, cz)
     auto harmonics = [&](const Stage& s, int buf, double cx, double cy, double cz) {
-        const double dx = px - cx, dy = py - cy, dz = pz - cz;
+        double dx = px - cx, dy = py - cy, dz = pz - cz;
         const bool real = jj < s.rows;
-        if constexpr (W == 0) {
+        if constexpr (W == 0 && !kPoly) {
             // a pad slot's position is stale (a row of an earlier chunk,
             // possibly of another structure): it enters the exp as d2 = 0
             const double d2 = fma(dz, dz, fma(dx, dx, dy * dy));
@@ -872,7 +881,41 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
         // the seed of its harmonics
         double seed = real ? 1.0 : 0.0;
         if constexpr (kWeighted) seed = real ? s.w : 0.0;
+        if constexpr (kPoly) {
+            // harmonics of the direction, times 4 pi w (soap.cpp:833-836)
+            const double radius = sqrt(dx * dx + dy * dy + dz * dz);
+            const double inverse = radius <= 1e-14 ? 0.0 : 1.0 / radius;
+            dx *= inverse;
+            dy *= inverse;
+            dz *= inverse;
+            seed *= 4.0 * 3.141592653589793238462643383279502884;
+        }
         harmonic_columns<LM, MLO, MHI>(dx, dy, dz, seed, comp, s_y + buf * PL::YWORDS + jj);
+    };
+
+    // Polynomial basis: the radial functions of a chunk's step groups, as the
+    // exp registers hold them, loaded a chunk ahead (a group past the chunk's
+    // loads its first)
+    double pre[kPoly ? GROUPS : 1][ND > 0 ? ND : 1][RPL];
+    auto load_radial = [&](const Stage& s) {
+        if constexpr (kPoly) {
+            const int groups = __builtin_amdgcn_readfirstlane(s.groups);
+            const double* rows = a.poly_g + uniform64(s.group) * (L * RPL * kWaveThreads) + lane;
+            unroll<GROUPS>([&](auto gc) {
+                constexpr int g = decltype(gc)::value;
+                const double* from = rows + (g < groups ? g : 0) * (L * RPL * kWaveThreads);
+                unroll<L>([&](auto lc) {
+                    constexpr int l = decltype(lc)::value;
+                    if constexpr ((kOwn >> l) & 1u) {
+                        constexpr int d = degrees_before(kOwn, l);
+                        unroll<RPL>([&](auto rc) {
+                            constexpr int rr = decltype(rc)::value;
+                            pre[g][d][rr] = from[(l * RPL + rr) * kWaveThreads];
+                        });
+                    }
+                });
+            });
+        }
     };
 
     // prologue: harmonics of the first chunk
@@ -886,6 +929,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
         }
     }
     load_positions(s1);
+    load_radial(s0);
     __syncthreads();
 
     int k = 0;
@@ -920,12 +964,16 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
             unroll<GROUPS>([&](auto gc) {
                 constexpr int g = decltype(gc)::value;
                 if (g >= groups0) return;
-                const double d2 = dbuf[GS * g];
                 double ev[ND > 0 ? ND : 1][RPL];
+                const double d2 = kPoly ? 0.0 : dbuf[GS * g];
                 unroll<ND>([&](auto dc) {
                     unroll<RPL>([&](auto rc) {
-                        ev[decltype(dc)::value][decltype(rc)::value] =
-                            exp_neg<ES == 4>(d2, e1[decltype(dc)::value][decltype(rc)::value], s_tab);
+                        constexpr int d = decltype(dc)::value, rr = decltype(rc)::value;
+                        if constexpr (kPoly) {
+                            ev[d][rr] = pre[g][d][rr];
+                        } else {
+                            ev[d][rr] = exp_neg<ES == 4>(d2, e1[d][rr], s_tab);
+                        }
                     });
                 });
                 unroll<L>([&](auto lc) {
@@ -945,6 +993,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
                 });
             });
         }
+        load_radial(s1);
         // a centre's sums end in the coefficient registers (an average
         // thereby sums per-centre coefficients, as a centre's row does)
         if (ends0) {
@@ -1018,24 +1067,25 @@ constexpr int ps_tiles(int ncr, bool summed) { return summed ? ncr : ncr * (ncr 
 // Wavefronts per SIMD a shape's registers are limited to: five (96 VGPRs)
 // where the widest wavefront's accumulators and coefficients leave room for
 // the rest (about 56 registers), else as many as they leave.
-template <int LM, int KG, int NCR>
+template <int LM, int KG, int NCR, int FORM>
 constexpr int block_waves_per_simd() {
     using PL = BlockPlan<LM, KG>;
-    int units = 0;
+    int registers = 0;
     for (int w = 0; w < PL::T; ++w) {
-        const int u = units_total(PL::own(w), PL::L);
-        units = u > units ? u : units;
+        // (a chunk's radial functions of the polynomial basis, loaded ahead)
+        const int ahead = FORM == kBlockPolynomial ? PL::GROUPS * popcount_c(PL::own(w)) * PL::RPL : 0;
+        const int r = 2 * (units_total(PL::own(w), PL::L) * (NCR + PL::RPL) + ahead) + 56;
+        registers = r > registers ? r : registers;
     }
-    const int registers = 2 * units * (NCR + PL::RPL) + 56;
     const int waves = 512 / ((registers + 7) / 8 * 8);
     return waves > 5 ? 5 : waves < 2 ? 2 : waves;
 }
 
 // Outer averages in LDS take four wavefronts per SIMD at most: their row in
 // LDS allows no more workgroups a CU, and with five the l_max 6 shape spills.
-template <int LM, int KG, int NCR, int ES, int MODE, bool kWeighted>
+template <int LM, int KG, int NCR, int ES, int MODE, int FORM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-    MODE == kBlockOuterLds && block_waves_per_simd<LM, KG, NCR>() > 4 ? 4 : block_waves_per_simd<LM, KG, NCR>()))) void
+    MODE == kBlockOuterLds && block_waves_per_simd<LM, KG, NCR, FORM>() > 4 ? 4 : block_waves_per_simd<LM, KG, NCR, FORM>()))) void
 k_soap_block(BlockArgs a) {
     using PL = BlockPlan<LM, KG>;
     // staging buffers, d2, exp table, padded S_lm table, power-spectrum
@@ -1057,6 +1107,11 @@ k_soap_block(BlockArgs a) {
     // the first rows of the second staging buffer, which the pad columns
     // of the first chunk read, start finite (zero); the exp table
     for (int i = tid; i < 3 * kYS; i += threads) s_y[PL::YWORDS + i] = 0.0;
+    // (and the second buffer's read the distances, which the polynomial
+    // basis does not stage)
+    if constexpr (FORM == kBlockPolynomial) {
+        for (int i = tid; i < 2 * kNb; i += threads) s_d2[i] = 0.0;
+    }
     for (int i = tid; i < kTab; i += threads) {
         const double t = exp2(static_cast<double>(i) / kTab);
         s_tab[i] = int2{__double2loint(t), __double2hiint(t) - (i << (20 - kTabBits))};
@@ -1083,15 +1138,15 @@ k_soap_block(BlockArgs a) {
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveThreads);
     if (wave == 0) {
-        block_role<LM, KG, NCR, ES, MODE, kWeighted, 0>(a, lds, s_ps, s_acc);
+        block_role<LM, KG, NCR, ES, MODE, FORM, 0>(a, lds, s_ps, s_acc);
     } else if constexpr (PL::T > 1) {
         if (wave == 1) {
-            block_role<LM, KG, NCR, ES, MODE, kWeighted, (PL::T > 1 ? 1 : 0)>(a, lds, s_ps, s_acc);
+            block_role<LM, KG, NCR, ES, MODE, FORM, (PL::T > 1 ? 1 : 0)>(a, lds, s_ps, s_acc);
         } else if constexpr (PL::T > 2) {
             if (wave == 2) {
-                block_role<LM, KG, NCR, ES, MODE, kWeighted, (PL::T > 2 ? 2 : 0)>(a, lds, s_ps, s_acc);
+                block_role<LM, KG, NCR, ES, MODE, FORM, (PL::T > 2 ? 2 : 0)>(a, lds, s_ps, s_acc);
             } else if constexpr (PL::T > 3) {
-                block_role<LM, KG, NCR, ES, MODE, kWeighted, (PL::T > 3 ? 3 : 0)>(a, lds, s_ps, s_acc);
+                block_role<LM, KG, NCR, ES, MODE, FORM, (PL::T > 3 ? 3 : 0)>(a, lds, s_ps, s_acc);
             }
         }
     }
@@ -1131,8 +1186,15 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
     using Inner = std::integral_constant<int, kBlockInner>;
     using Small = std::integral_constant<int, kBlockInnerSmall>;
     using Outer = std::integral_constant<int, kBlockOuterLds>;
-    using Plain = std::false_type;
-    using Weighted = std::true_type;
+    using Plain = std::integral_constant<int, kBlockPlain>;
+    using Weighted = std::integral_constant<int, kBlockWeighted>;
+    using Polynomial = std::integral_constant<int, kBlockPolynomial>;
+    if (a.poly_g != nullptr) {
+        if constexpr (KG <= kBlockPolyGroups) {
+            if (a.struct_offsets == nullptr) launch(F64{}, Rows{}, Polynomial{}); else launch(F64{}, Inner{}, Polynomial{});
+        }
+        return;
+    }
     const bool f32 = a.table_dtype == 4, weighted = a.row_w_mask != 0;
     if constexpr (kEveryForm) {
         // reading a weight of 1 per row costs the unweighted forms 2-4 %

@@ -26,6 +26,7 @@ struct MfmaDims {
     int crow;
     int radial;      // 0 GTO, 1 polynomial
     int grid;        // polynomial radial grid points
+    int64_t poly_first; // polynomial: first centre of the slice poly_g holds
     int weighted;    // 1 when any neighbour weight can differ from 1
     int weighting;   // 0 none, 1 poly, 2 pow, 3 exp
     int has_w0;
@@ -52,8 +53,8 @@ struct MfmaTables {
     const int32_t* fbase;
     const int32_t* fstride;
     const double* species_w;  // species weights [S]
-    const double* poly_bw;    // polynomial: w_q r_q^2 g_k(r_q), [q * n + k]
-    const double* poly_grid;  // polynomial: r_q
+    const double* poly_g;     // polynomial: radial functions of the slice's pair rows (launch_poly_radial)
+    const int64_t* poly_start; // polynomial: the graph's first row of each centre
     const int32_t* bin_atom;  // atom of each binned image (exact-self test for w0)
     const int32_t* bin_image; // image of each binned image
     const ImageDesc* images;  // image table (integer shifts)
@@ -130,10 +131,29 @@ void launch_quad_expand(hipStream_t stream, int waves, int kg, int instr, const 
 inline int mfma_coefficient_rows(int Sc, int n, int compression) { return Sc * n + (compression == 2 ? n : 0) + 1; }
 int mfma_padded_row(int l_max);
 size_t mfma_lds_bytes(const MfmaDims& d);
+// LDS a polynomial plan must leave free beside that (once the radial kernels
+// of a grid step): the limit on its shape
+inline size_t mfma_plan_reserve(const MfmaDims& d) {
+    return d.radial == 1 ? static_cast<size_t>(d.L) * 32 * 4 * sizeof(double) : 0;
+}
 void launch_mfma_expand(hipStream_t stream, int template_tiles, const PreparedBatch& pb, const DeviceGraph& g,
                         const MfmaTables& tab, const MfmaDims& d, const int64_t* item_begin, int64_t base,
                         int64_t count, void* out, int64_t pitch, double* partial);
 void launch_mfma_finalize(hipStream_t stream, const PreparedBatch& pb, const MfmaTables& tab, const MfmaDims& d,
                           const double* partial, const int64_t* struct_items, void* out, int64_t pitch);
+
+
+// Radial functions of the polynomial basis (soap_poly.hip) of every pair row
+// of centres [first, first + count): out[(row - first row of centre `first`)
+// * L n + l n + k], or with step_groups != 0 (one or two radial groups) as the
+// register-coefficient kernel reads them (BlockArgs::poly_g), step_groups
+// groups a centre.  tables: poly_radial_tables on the device (r_q, 1 / r_q,
+// the weighted basis w_q r_q^2 g_k(r_q) at 4 poly_channel_groups(n) channels
+// a point, padded to whole steps of four points; then the rows of a pair at
+// distance zero).  bw is the weighted basis, [q * n + k].
+int poly_channel_groups(int n);
+std::vector<double> poly_radial_tables(int grid, int n, double eta, const double* points, const std::vector<double>& bw);
+void launch_poly_radial(hipStream_t stream, const PreparedBatch& pb, const DeviceGraph& g, const double* tables,
+                        const MfmaDims& d, int64_t first, int64_t count, int64_t step_groups, double* out);
 
 } // namespace mdx

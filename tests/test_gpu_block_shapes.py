@@ -17,7 +17,7 @@ import pytest
 
 from conftest import scaled_error
 from mdescriptor_amd import _hip
-from mdescriptor_amd.descriptors.basis import basis_gto
+from mdescriptor_amd.descriptors.basis import basis_gto, basis_polynomial
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +102,35 @@ def test_outer_average_past_the_lds_row(hip_context, oracle):
     than 48 KB): a float64 partial row per centre."""
 
     _check(hip_context, oracle, _structures(5, (21, 13, 1, 20), SPECIES[:5]), (5, 9, 8), "outer", "float64")
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 1, 2), (4, 4, 3), (5, 3, 7), (2, 5, 2), (4, 5, 5), (5, 5, 6), (3, 4, 9),  # radial functions in step groups
+    (2, 4, 1), (3, 3, 10),                                             # by row, for the 16x16 kernel
+])
+@pytest.mark.parametrize("average", ["off", "inner", "outer"])
+@pytest.mark.parametrize("name", ["default", "pow_w0", "mu1nu1"])
+def test_polynomial_basis(hip_context, oracle, shape, average, name):
+    """Radial functions computed before the expansion, for the kernel that
+    reads them in step groups and for the one that reads them by row; a lone
+    atom (only the pair at distance zero), weights and a compression."""
+
+    count, n_max, l_max = shape
+    species = SPECIES[:count]
+    options = {"default": {}, "pow_w0": dict(POW_W0), "mu1nu1": {"compression": "mu1nu1"}}[name]
+    options["polynomial"] = basis_polynomial(4.0, n_max)
+    for sizes, dtype in (((21, 13, 1, 20), "float64"), ((70, 66), "float32")):
+        batch = _structures(sum(shape), sizes, species)
+        arguments = dict(species=species, n_max=n_max, l_max=l_max, r_cut=4.0, sigma=1.0, alphas=None, betas=None,
+                         average=average, options=options)
+        plan = _hip.SoapPlan(hip_context, dtype=dtype, **arguments)
+        try:
+            values, timing = plan.compute(batch)
+        finally:
+            plan.close()
+        assert (timing["expansion_tiles"] <= -1000) == (2 <= l_max <= 9)
+        expected = oracle.soap(batch, **arguments)
+        assert values.shape == expected.shape
+        assert np.all(np.isfinite(values))
+        error = scaled_error(values, expected)
+        assert error <= GATES[dtype], f"{shape} {average} {dtype} {name}: scaled error {error:.3e}"
