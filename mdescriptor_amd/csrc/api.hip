@@ -268,6 +268,38 @@ void run_pipeline(mdx_hip_ctx* ctx, const mdx_soap_plan& plan, mdx::PreparedBatc
     }
 }
 
+// Device bytes a batch holds.
+size_t batch_bytes(mdx_device_batch& b) {
+    size_t bytes = b.partials.bytes + b.partials2.bytes;
+    auto add = [&](mdx::DeviceBuffer& buffer) { bytes += buffer.bytes; };
+    b.pb.for_each_buffer(add);
+    b.graph.for_each_buffer(add);
+    b.graph2.for_each_buffer(add);
+    return bytes;
+}
+
+// Waits for the context's streams, which may still work on the batch, and
+// clears what belongs to its caller, so that another upload may take its
+// buffers.
+bool reset_batch(mdx_device_batch& b, const hipStream_t streams[3]) {
+    for (int i = 0; i < 3; ++i) {
+        if (hipStreamSynchronize(streams[i]) != hipSuccess) return false;
+    }
+    b.pb2.reset();
+    b.queued[0] = b.queued[1] = false;
+    b.next_set = 0;
+    b.pending = -1;
+    b.pending_plan = nullptr;
+    b.pending_out = nullptr;
+    b.pending_cancel = nullptr;
+    for (mdx::DeviceGraph* g : {&b.graph, &b.graph2}) {
+        g->slot_cap = mdx::kMinSlotCap;
+        g->stats_pending = false;
+    }
+    b.spare.reset();
+    return true;
+}
+
 // True for memory from hipHostMalloc (page-locked, DMA-able at full PCIe
 // rate); pageable memory reports "unregistered" or an error, which is cleared.
 bool is_pinned_host(const void* p) {
@@ -375,6 +407,63 @@ void download_result(mdx_hip_ctx* ctx, const void* src, int64_t rows, int64_t ro
 
 } // namespace
 
+namespace mdx {
+
+mdx_device_batch* SpareBatch::take() {
+    std::lock_guard<std::mutex> lock(mutex);
+    mdx_device_batch* b = batch;
+    batch = nullptr;
+    return b;
+}
+
+bool SpareBatch::keep(mdx_device_batch* returned) {
+    if (batch_bytes(*returned) > kSpareBytes) return false;
+    mdx_device_batch* old = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(mutex); // (the context waits for it before its streams go)
+        if (!open || !reset_batch(*returned, streams)) return false;
+        old = batch;
+        batch = returned;
+    }
+    delete old;
+    return true;
+}
+
+bool SpareBatch::drop() {
+    mdx_device_batch* b = take();
+    delete b;
+    return b != nullptr;
+}
+
+SpareBatch::~SpareBatch() { delete batch; }
+
+namespace {
+std::mutex g_spares_mutex;
+std::vector<std::weak_ptr<SpareBatch>> g_spares;
+} // namespace
+
+void register_spare(const std::shared_ptr<SpareBatch>& spare) {
+    std::lock_guard<std::mutex> lock(g_spares_mutex);
+    g_spares.erase(std::remove_if(g_spares.begin(), g_spares.end(), [](const auto& w) { return w.expired(); }),
+                   g_spares.end());
+    g_spares.push_back(spare);
+}
+
+bool drop_spare_batches() {
+    std::vector<std::shared_ptr<SpareBatch>> spares;
+    {
+        std::lock_guard<std::mutex> lock(g_spares_mutex);
+        for (const auto& w : g_spares) {
+            if (auto s = w.lock()) spares.push_back(std::move(s));
+        }
+    }
+    bool dropped = false;
+    for (const auto& s : spares) dropped = s->drop() || dropped;
+    return dropped;
+}
+
+} // namespace mdx
+
 extern "C" {
 
 int mdx_hip_host_alloc(size_t bytes, void** out) {
@@ -415,9 +504,14 @@ int mdx_hip_create(int device, mdx_hip_ctx** out) {
         try {
             DeviceScope scope(device);
             ctx->device = device;
+            ctx->spare = std::make_shared<mdx::SpareBatch>();
+            mdx::register_spare(ctx->spare);
             MDX_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
             MDX_HIP(hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking));
             MDX_HIP(hipStreamCreateWithFlags(&ctx->graph_stream, hipStreamNonBlocking));
+            ctx->spare->streams[0] = ctx->stream;
+            ctx->spare->streams[1] = ctx->copy_stream;
+            ctx->spare->streams[2] = ctx->graph_stream;
             for (auto& ev : ctx->events) MDX_HIP(hipEventCreate(&ev));
             for (auto& ev : ctx->stage_events) MDX_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
             for (auto& ev : ctx->list_events) MDX_HIP(hipEventCreate(&ev));
@@ -466,6 +560,13 @@ void mdx_hip_destroy(mdx_hip_ctx* ctx) {
         }
         if (ctx->pinned != nullptr) (void)hipHostFree(ctx->pinned);
         ctx->pinned = nullptr;
+    }
+    if (ctx->spare) {
+        {
+            std::lock_guard<std::mutex> lock(ctx->spare->mutex);
+            ctx->spare->open = false;
+        }
+        ctx->spare->drop();
     }
     hipStream_t stream = ctx->stream;
     hipStream_t copy_stream = ctx->copy_stream;
@@ -806,9 +907,11 @@ int mdx_hip_batch_upload(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_
         if (plan == nullptr || batch == nullptr) throw mdx::Error(MDX_INVALID_ARGUMENT, "null plan or batch");
         if (plan->device != ctx->device) throw mdx::Error(MDX_INVALID_ARGUMENT, "plan belongs to another device");
         DeviceScope scope(ctx->device);
-        auto db = new mdx_device_batch();
+        mdx_device_batch* db = ctx->spare->take();
+        if (db == nullptr) db = new mdx_device_batch();
         try {
             db->device = ctx->device;
+            db->spare = ctx->spare;
             db->pb.include_boundary = 1;
             mdx::prepare_batch(*batch, plan->species.data(), plan->S, plan->cutoff, db->pb);
             mdx::upload_batch(ctx->stream, *batch, db->pb);
@@ -904,7 +1007,8 @@ void mdx_hip_batch_destroy(mdx_device_batch* batch) {
     int previous = -1;
     (void)hipGetDevice(&previous);
     (void)hipSetDevice(batch->device);
-    delete batch;
+    const std::shared_ptr<mdx::SpareBatch> spare = batch->spare;
+    if (!spare || !spare->keep(batch)) delete batch;
     if (previous >= 0) (void)hipSetDevice(previous);
 }
 

@@ -72,7 +72,13 @@ void DeviceBuffer::reserve(size_t size) {
     }
     release();
     const size_t rounded = std::max<size_t>(256, (size + 255) & ~size_t(255));
-    MDX_HIP(hipMalloc(&ptr, rounded));
+    hipError_t code = hipMalloc(&ptr, rounded);
+    if (code == hipErrorOutOfMemory && drop_spare_batches()) {
+        (void)hipGetLastError();
+        code = hipMalloc(&ptr, rounded);
+    }
+    if (code != hipSuccess) ptr = nullptr;
+    check_hip(code, "hipMalloc(&ptr, rounded)");
     bytes = rounded;
 }
 

@@ -266,6 +266,14 @@ struct PreparedBatch {
     DeviceBuffer d_atom_rank;    // i32[atoms]: place among its home cell's centres
     PinnedWords frame_host;      // the summary, read back
     StreamPoint frame_read;
+    template <typename F> void for_each_buffer(F f) {
+        for (DeviceBuffer* b : {&d_positions, &d_types, &d_atom_struct, &d_geom, &d_images, &d_offsets, &d_frame,
+                                &d_frame_items, &d_frame_item_start, &d_frame_lists, &d_struct_cells, &d_struct_chunks,
+                                &d_cell_lists, &d_struct_list, &d_cell_centres, &d_atom_cell, &d_atom_home,
+                                &d_atom_rank}) {
+            f(*b);
+        }
+    }
 };
 
 // Device graph (kernel 1 output).  Pairs are indices into the cell-sorted
@@ -420,8 +428,35 @@ void fill_neighbor_list(hipStream_t stream, const PreparedBatch& pb, const Devic
 } // namespace mdx
 
 // Opaque C-ABI objects.
+struct mdx_device_batch;
+
+namespace mdx {
+// The last batch destroyed on a context, kept with its device buffers (at
+// most kSpareBytes) for the next upload: a call that uploads a batch, runs it
+// and destroys it (SOAP.compute_into) then allocates nothing after the first
+// (35 device and two pinned allocations and their frees, 0.3 ms a call, up to
+// 1.6 ms for 20,000 structures).  Idle: its work has finished, and it belongs
+// to no caller.  Freed with the context, or when a device allocation fails.
+struct SpareBatch {
+    std::mutex mutex;
+    bool open = true; // false once the context is going
+    hipStream_t streams[3] = {}; // the context's
+    mdx_device_batch* batch = nullptr;
+    mdx_device_batch* take();              // the spare (the caller's now), or null
+    bool keep(mdx_device_batch* returned); // false: not kept (the caller deletes it)
+    bool drop();                           // frees the spare; true if there was one
+    ~SpareBatch();
+};
+constexpr size_t kSpareBytes = size_t(1) << 30;
+// Every context's spare freed; true if memory came back (device allocations
+// retry then).
+bool drop_spare_batches();
+void register_spare(const std::shared_ptr<SpareBatch>& spare);
+} // namespace mdx
+
 struct mdx_hip_ctx {
     int device = 0;
+    std::shared_ptr<mdx::SpareBatch> spare; // shared with the batches uploaded on this context
     hipStream_t stream = nullptr;
     std::mutex mutex;
     std::string last_error;
@@ -513,6 +548,7 @@ struct mdx_device_batch {
     // is built and expanded again if a centre overflowed its slot) by the next
     // call on the batch: its set (-1: none), plan, output and cancel flag.
     int pending = -1;
+    std::shared_ptr<mdx::SpareBatch> spare; // the context's, which takes the batch back when it is destroyed
     const mdx_soap_plan* pending_plan = nullptr;
     void* pending_out = nullptr;
     int64_t pending_pitch = 0;

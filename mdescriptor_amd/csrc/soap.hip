@@ -66,6 +66,9 @@ int64_t run_centres(const PreparedBatch& pb, size_t width, int64_t budget) {
     return std::min<int64_t>(length, kItemCentres);
 }
 
+// Pair rows of the graph's layout.
+int64_t graph_rows(const PreparedBatch& pb, const DeviceGraph& g) { return g.slots > 0 ? pb.atoms * g.slots : g.pairs; }
+
 struct SoapDims {
     int S, n, l_max, L, H, LN, CH;
     int mode;      // 0 off, 1 inner, 2 outer
@@ -507,7 +510,7 @@ Fold fold_of(int64_t most_items) {
 
 // Scratch of a run: its partial rows, folded rows, item tables and row weights.
 size_t scratch_bytes(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g, const Choice& c) {
-    size_t bytes = c.block && p.weighted != 0 ? (g.pair_bin.bytes / sizeof(uint32_t)) * sizeof(double) + 256 : 0;
+    size_t bytes = c.block && p.weighted != 0 ? static_cast<size_t>(graph_rows(pb, g)) * sizeof(double) + 256 : 0;
     if (p.average == 0 || !c.partials()) return bytes;
     const int64_t run = c.block_outer ? 1 : c.run;
     int64_t items = 0, most = 0;
@@ -590,7 +593,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     // weight, computed once before the expansion (k_block_row_weights), after
     // any partial rows in the scratch buffer
     const size_t row_w_bytes =
-        block && p.weighted != 0 ? ((g.pair_bin.bytes / sizeof(uint32_t)) * sizeof(double) + 255) & ~size_t(255) : 0;
+        block && p.weighted != 0 ? (static_cast<size_t>(graph_rows(pb, g)) * sizeof(double) + 255) & ~size_t(255) : 0;
     double* d_row_w = nullptr;
     // polynomial basis: the radial functions of a slice of centres, beside
     // any partial rows and row weights

@@ -485,3 +485,40 @@ def test_pipelined_frames_share_one_output(hip_context, oracle):
     finally:
         resident.close()
         plan.close()
+
+
+def test_destroyed_batches_leave_nothing_to_the_next(hip_context, oracle):
+    """A destroyed batch's buffers serve the next upload: batches of other
+    sizes, plans, averages and layouts in turn (one with pipelined frames
+    still queued, one after a context of its own), each against the oracle."""
+
+    other = _hip.Context(0)
+    kept = []
+    for number, (config, average) in enumerate([(2, "inner"), (1, "off"), (3, "outer"), (2, "off"), (3, "inner"),
+                                                (1, "outer")]):
+        work = workloads.config(config, "small")
+        p = work.params
+        context = other if number == 3 else hip_context
+        alphas, betas = basis_gto(p["r_cut"], p["n_max"], p["l_max"])
+        plan = _hip.SoapPlan(context, species=p["species"], n_max=p["n_max"], l_max=p["l_max"], r_cut=p["r_cut"],
+                             sigma=1.0, alphas=alphas, betas=betas, average=average, dtype="float64")
+        expected = oracle.soap(work.batch, species=p["species"], n_max=p["n_max"], l_max=p["l_max"],
+                               r_cut=p["r_cut"], sigma=1.0, alphas=alphas, betas=betas, average=average)
+        out = _hip.DeviceMemory(expected.nbytes)
+        batch = _hip.DeviceBatch(plan, work.batch)
+        batch.run(out.address, expected.shape[1] * 8)
+        values = out.to_host(np.empty_like(expected))
+        assert scaled_error(values, expected) <= F64_GATE, (config, average)
+        if number % 2 == 0:
+            # frames still queued when the batch goes
+            for _ in range(3):
+                batch.run_frame(work.batch.positions, out.address, expected.shape[1] * 8)
+        if number == 3:
+            kept.append((batch, plan))  # outlive their context
+            continue
+        batch.close()
+        plan.close()
+    other.close()
+    for batch, plan in kept:
+        batch.close()
+        plan.close()
