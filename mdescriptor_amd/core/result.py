@@ -54,6 +54,24 @@ def owned_values(array: np.ndarray) -> _OwnedValues:
     return _OwnedValues(array)
 
 
+class _OwnedSamples(_OwnedValues):
+    """Fresh int64 pair samples of the plugin that the result may keep without
+    a copy: the device forms them from the batch's own offsets (every index is
+    in range by construction), so the result checks their shape only.
+    Checking and copying 1.2 million of them took 18 of a call's 21 ms."""
+
+    __slots__ = ()
+
+    def __init__(self, array: Any) -> None:
+        super().__init__(array)
+        if array.dtype != np.int64:
+            raise TypeError("owned pair samples must be int64")
+
+
+def owned_samples(array: np.ndarray) -> _OwnedSamples:
+    return _OwnedSamples(array)
+
+
 def format_values(values: Any, *, dtype: str = "float64", sparse: bool = False) -> Any:
     """Dense array of ``dtype`` or, with ``sparse``, a CSR matrix (result.py:64-87)."""
 
@@ -239,10 +257,14 @@ class DescriptorResult:
                 samples = atom_samples(offsets)
             else:
                 raise ValueError("pair-level results require explicit pair samples")
-        samples = np.asarray(samples)
-        if samples.size and not np.issubdtype(samples.dtype, np.integer):
-            raise ValueError("samples must contain integer indices")
-        samples = np.array(samples, dtype=np.int64, order="C", copy=True)
+        checked = isinstance(samples, _OwnedSamples)
+        if checked:
+            samples = samples.array
+        else:
+            samples = np.asarray(samples)
+            if samples.size and not np.issubdtype(samples.dtype, np.integer):
+                raise ValueError("samples must contain integer indices")
+            samples = np.array(samples, dtype=np.int64, order="C", copy=True)
         expected = {DescriptorLevel.STRUCTURE: 1, DescriptorLevel.ATOM: 2, DescriptorLevel.PAIR: 6}[level]
         if samples.ndim != 2 or samples.shape != (rows, expected):
             raise ValueError(f"{level.value}-level samples must have shape (rows, {expected})")
@@ -250,6 +272,7 @@ class DescriptorResult:
             # result.py:399-410: structure and both local atom indices in range
             if atom_offsets is None:
                 raise ValueError("pair-level results require atom row offsets for sample validation")
+        if level is DescriptorLevel.PAIR and not checked:
             if rows and (np.any(samples[:, :3] < 0) or np.any(samples[:, 0] >= len(offsets) - 1)):
                 raise ValueError("pair samples contain an invalid structure or atom index")
             counts = np.diff(atom_offsets)
@@ -295,6 +318,7 @@ __all__ = [
     "atom_samples",
     "format_values",
     "metadata_envelope",
+    "owned_samples",
     "owned_values",
     "structure_samples",
 ]

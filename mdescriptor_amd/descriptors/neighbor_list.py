@@ -34,7 +34,7 @@ from ..core.backends import HipBackend
 from ..core.descriptor import Descriptor
 from ..core.errors import DescriptorConfigError, DescriptorInputError
 from ..core.options import CONFIGURATION_SCHEMA_VERSION, ExecutionOptions, OutputOptions, coerce_options
-from ..core.result import DescriptorResult, format_values, metadata_envelope, owned_values
+from ..core.result import DescriptorResult, format_values, metadata_envelope, owned_samples, owned_values
 
 SUPPORTED_DEVICES = ("hip",)
 LABELS = ("dx", "dy", "dz", "distance")
@@ -132,7 +132,7 @@ class NeighborList(Descriptor):
             values = owned_values(values)
         metadata = self._envelope()
         result = DescriptorResult(values, "pair", batch.ids, raw["row_offsets"], LABELS, metadata,
-                                  samples=raw["samples"], feature_count=self.feature_count,
+                                  samples=owned_samples(raw["samples"]), feature_count=self.feature_count,
                                   _atom_row_offsets=np.asarray(batch.offsets, dtype=np.int64))
         self._metadata_snapshot = metadata
         return result

@@ -373,3 +373,24 @@ def test_batch_field_conversion_messages():
         with pytest.raises(ValueError, match=message) as info:
             mdx.StructureBatch(**kwargs)
         assert list(info.value.path) == ["input", field]
+
+
+def test_owned_pair_samples_are_kept_and_checked_for_shape():
+    """Samples handed over by the plugin are kept without a copy, read-only;
+    any others are copied and checked index by index."""
+
+    from mdescriptor_amd.core.result import DescriptorResult, owned_samples, owned_values
+
+    samples = np.array([[0, 0, 1, 0, 0, 0], [0, 1, 0, 0, 0, 0]], dtype=np.int64)
+    build = lambda s: DescriptorResult(owned_values(np.zeros((2, 4))), "pair", ("a",), [0, 2],  # noqa: E731
+                                       ("dx", "dy", "dz", "distance"), samples=s, _atom_row_offsets=np.array([0, 2]))
+    result = build(owned_samples(samples))
+    assert result.samples is samples and not result.samples.flags.writeable
+    copied = build(samples.tolist())
+    np.testing.assert_array_equal(copied.samples, samples)
+    with pytest.raises(ValueError, match="shape"):
+        build(owned_samples(np.zeros((3, 6), dtype=np.int64)))
+    with pytest.raises(TypeError, match="int64"):
+        owned_samples(np.zeros((2, 6), dtype=np.int32))
+    with pytest.raises(ValueError, match="invalid"):
+        build([[0, 0, 2, 0, 0, 0], [0, 1, 0, 0, 0, 0]])
