@@ -699,8 +699,10 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     };
 
     const int64_t F = a.F;
-    // float32 rows of a plan whose tables are those of float64 rows
-    const bool half_rows = ES == 8 && a.out_bytes == 4;
+    // float32 rows of a plan whose tables are those of float64 rows (never the
+    // unweighted form, which is compiled with float32 tables too: the choice
+    // per store cost its float64 rows 1-2 %)
+    const bool half_rows = ES == 8 && FORM != kBlockPlain && a.out_bytes == 4;
     // row end: C <- (S_lm C)^T beta^T scaled by scale0, the power spectrum of
     // the owned degrees to output row row0, and C back to zero
     auto row_end = [&](int64_t row0, double scale0) {
