@@ -175,6 +175,8 @@ int mdx_hip_soap_compute(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_
  * (the H2D part of Backend::compute, cpp/cuda/src/backend.cu:353-356) */
 int mdx_hip_batch_upload(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_batch_view* batch,
                          mdx_device_batch** out);
+/* The context keeps one destroyed batch's buffers (at most 1 GiB) for the next
+ * upload; they are freed with the context or when an allocation fails. */
 void mdx_hip_batch_destroy(mdx_device_batch* batch);
 
 /* New positions for a device-resident batch (a new frame of the same system:
@@ -208,9 +210,12 @@ int mdx_hip_soap_run(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, mdx_device_bat
 /* mdx_hip_soap_run without device allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory during the run
  * (tight serving loops, code that must not call hipMalloc).  Same arguments,
- * kernels and results as mdx_hip_soap_run; the run's scratch (neighbour graph,
+ * results as mdx_hip_soap_run; the run's scratch (neighbour graph,
  * partial sums of the averaged modes) lives in one static device array of
  * MDX_NOALLOC_SCRATCH_BYTES per device instead of buffers owned by the batch.
+ * Averages whose partial rows do not fit beside the graph take longer runs of
+ * centres, then a workgroup per structure or a kernel with smaller rows: the
+ * same features up to rounding.
  * The plan, the batch and out_device are the caller's, made beforehand.  A
  * batch whose scratch does not fit returns MDX_INVALID_ARGUMENT with a message
  * that names the maximum.  All contexts on one device share its array, which
