@@ -602,17 +602,12 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                : item_begin_h.empty() ? item
                                       : item_begin_h[static_cast<size_t>(item)];
     };
-    int64_t poly_centres = 0, step_groups = 0;
+    int64_t poly_centres = 0;
     size_t poly_bytes = 0;
+    PolyLayout layout;
     if (p.radial_basis == 1) {
-        const int64_t rows = std::max<int64_t>(1, g.row_bound);
-        int64_t centre_bytes = rows * p.L * p.n * static_cast<int64_t>(sizeof(double));
-        if (block) {
-            // every species' rows padded to whole step groups
-            const int64_t slots = p.block_kg == 2 ? 8 : 16;
-            step_groups = rows / slots + p.S;
-            centre_bytes = step_groups * p.L * kWave * static_cast<int64_t>(sizeof(double));
-        }
+        layout = poly_layout(g.row_bound, p.S, p.L, p.n, block);
+        const int64_t centre_bytes = layout.centre * static_cast<int64_t>(sizeof(double));
         int64_t room = kPolySliceBytes;
         if (partials.arena != nullptr) {
             const size_t left = partials.arena->left() + partials.bytes, used = scratch_bytes(p, pb, g, choice) + 4096;
@@ -731,7 +726,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         tab.fstride = p.d_fstride.as<int32_t>();
         tab.species_w = p.d_species_w.as<double>();
         tab.poly_g = d_poly;
-        tab.poly_start = g.pair_start.as<int64_t>();
+        tab.poly_centre = layout.centre;
         tab.bin_atom = g.bin_atom.as<int32_t>();
         tab.bin_image = g.bin_image.as<int32_t>();
         tab.images = pb.d_images.as<ImageDesc>();
@@ -782,7 +777,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                 for (count = 1; count < most && first_centre(base + count + 1) - first <= poly_centres;) ++count;
                 md.poly_first = first;
                 launch_poly_radial(stream, pb, g, p.d_poly.as<double>(), md, first, first_centre(base + count) - first,
-                                   step_groups, d_poly);
+                                   layout, d_poly, static_cast<int64_t>(poly_bytes / sizeof(double)));
             }
             if (block) {
                 BlockArgs ba{};
@@ -816,7 +811,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                 ba.row_w_mask = p.weighted != 0 ? -1 : 0;
                 ba.poly_g = d_poly;
                 ba.poly_first = md.poly_first;
-                ba.poly_groups = step_groups;
+                ba.poly_groups = layout.groups;
                 ba.out = block_outer ? static_cast<void*>(d_partial) : out_device;
                 ba.pitch = block_outer ? static_cast<int64_t>(partial_width * sizeof(double)) : pitch_bytes;
                 block_args = ba;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "mdx_internal.h"
+#include "poly_layout.h"
 
 namespace mdx {
 
@@ -54,7 +55,7 @@ struct MfmaTables {
     const int32_t* fstride;
     const double* species_w;  // species weights [S]
     const double* poly_g;     // polynomial: radial functions of the slice's pair rows (launch_poly_radial)
-    const int64_t* poly_start; // polynomial: the graph's first row of each centre
+    int64_t poly_centre;      // polynomial: doubles a centre in poly_g (PolyLayout)
     const int32_t* bin_atom;  // atom of each binned image (exact-self test for w0)
     const int32_t* bin_image; // image of each binned image
     const ImageDesc* images;  // image table (integer shifts)
@@ -144,16 +145,18 @@ void launch_mfma_finalize(hipStream_t stream, const PreparedBatch& pb, const Mfm
 
 
 // Radial functions of the polynomial basis (soap_poly.hip) of every pair row
-// of centres [first, first + count): out[(row - first row of centre `first`)
-// * L n + l n + k], or with step_groups != 0 (one or two radial groups) as the
-// register-coefficient kernel reads them (BlockArgs::poly_g), step_groups
-// groups a centre.  tables: poly_radial_tables on the device (r_q, 1 / r_q,
+// of centres [first, first + count), at the layout's places in out: by row l n
+// + k of a pair row's values, or in step groups (one or two radial groups) as
+// the register-coefficient kernel reads them (BlockArgs::poly_g).  out holds
+// `capacity` doubles; a slice that needs more is refused before the launch.
+// tables: poly_radial_tables on the device (r_q, 1 / r_q,
 // the weighted basis w_q r_q^2 g_k(r_q) at 4 poly_channel_groups(n) channels
 // a point, padded to whole steps of four points; then the rows of a pair at
 // distance zero).  bw is the weighted basis, [q * n + k].
 int poly_channel_groups(int n);
 std::vector<double> poly_radial_tables(int grid, int n, double eta, const double* points, const std::vector<double>& bw);
 void launch_poly_radial(hipStream_t stream, const PreparedBatch& pb, const DeviceGraph& g, const double* tables,
-                        const MfmaDims& d, int64_t first, int64_t count, int64_t step_groups, double* out);
+                        const MfmaDims& d, int64_t first, int64_t count, const PolyLayout& layout, double* out,
+                        int64_t capacity);
 
 } // namespace mdx

@@ -320,7 +320,7 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
                 if constexpr (kPoly) {
                     // the radial functions of the chunk's rows (pad slots, whose
                     // harmonics are zero, and the pad entry: zero)
-                    const double* rows = tab.poly_g + (centre_pairs - tab.poly_start[d.poly_first]) * (L * n);
+                    const double* rows = tab.poly_g + poly_row(tab.poly_centre, centre, d.poly_first, 0, L * n);
 #pragma unroll 4
                     for (int s = wave; s < kNb; s += T) {
                         int q;

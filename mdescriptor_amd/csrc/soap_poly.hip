@@ -54,9 +54,7 @@ struct PolyArgs {
     int64_t first, count; // centres [first, first + count)
     int split;            // workgroups per centre, or
     int share;            // centres per workgroup (1, 2 or kWaves)
-    // layout of out: 0 a row of L n values per pair; else the register-
-    // coefficient kernel's step groups, groups of them a centre
-    int64_t groups;
+    PolyLayout layout; // of out
     double* out;
 };
 
@@ -103,7 +101,7 @@ __global__ __launch_bounds__(kThreads) void k_poly_radial(PolyArgs a) {
     const int per_centre = kWaves / a.share; // wavefronts of a centre here
     const int64_t offset = static_cast<int64_t>(block) * a.share + wave / per_centre;
     const int64_t c = a.first + min(offset, a.count - 1);
-    constexpr int R = KG == 2 ? 2 : 1, GS = 16 / R; // slots of a step group
+    constexpr int R = KG == 2 ? 2 : 1, GS = poly_group_slots(KG); // slots of a step group
     const int tile = part * kWaves + wave % per_centre;
     int groups = 0; // the centre's step groups: every species' rows in whole ones
     for (int t = 0; t < a.S; ++t) groups += (a.counts[c * a.S + t] + GS - 1) / GS;
@@ -204,13 +202,13 @@ __global__ __launch_bounds__(kThreads) void k_poly_radial(PolyArgs a) {
     const int row = 4 * ((lane / 4) % 4) + lane / 16;
     const bool own = ((__ballot(at_centre) >> row) & 1) != 0;
     const int pair = slot_row(row);
-    if (a.groups != 0) {
+    if (a.layout.groups != 0) {
         // 16 lanes per neighbour of a step, 4 per block of a radial group
         // and step phase, one per channel; zero past the species' rows
         if (R * tile + row / GS >= groups) return;
         const int s = row % GS;
-        double* out = a.out + ((c - a.first) * a.groups + R * tile + row / GS) * (a.L * (KG / R) * kWave) + s % 4 * 16 +
-                      s / 4 * R * 4 + lane % 4;
+        double* out = a.out + poly_group(a.layout.groups, c, a.first, R * tile + row / GS, a.L * (KG / R) * kWave) +
+                      s % 4 * 16 + s / 4 * R * 4 + lane % 4;
 #pragma unroll
         for (int l = 0; l < LD; ++l) {
 #pragma unroll
@@ -221,7 +219,7 @@ __global__ __launch_bounds__(kThreads) void k_poly_radial(PolyArgs a) {
             }
         }
     } else if (pair >= 0) {
-        double* out = a.out + (first_row - a.pair_start[a.first] + pair) * (a.L * a.n);
+        double* out = a.out + poly_row(a.layout.centre, c, a.first, pair, a.L * a.n);
 #pragma unroll
         for (int l = 0; l < LD; ++l) {
 #pragma unroll
@@ -278,8 +276,12 @@ std::vector<double> poly_radial_tables(int grid, int n, double eta, const double
 }
 
 void launch_poly_radial(hipStream_t stream, const PreparedBatch& pb, const DeviceGraph& g, const double* tables,
-                        const MfmaDims& d, int64_t first, int64_t count, int64_t step_groups, double* out) {
+                        const MfmaDims& d, int64_t first, int64_t count, const PolyLayout& layout, double* out,
+                        int64_t capacity) {
     if (count <= 0) return;
+    if (out == nullptr || count * layout.centre > capacity) {
+        throw Error(MDX_INTERNAL, "radial functions of a slice of centres outgrow their scratch");
+    }
     const int groups = poly_channel_groups(d.n);
     const int64_t padded = (d.grid + 3) / 4 * 4;
     PolyArgs a{};
@@ -301,13 +303,13 @@ void launch_poly_radial(hipStream_t stream, const PreparedBatch& pb, const Devic
     a.steps = static_cast<int>(padded / 4);
     a.first = first;
     a.count = count;
-    a.groups = step_groups;
+    a.layout = layout;
     a.out = out;
     // a wavefront per tile, as many as the centres' rows can fill: workgroups
     // past them end at once, and the device balances the others (a workgroup
     // per centre left a second round of workgroups a quarter full: 451 us
     // against 405 for 834,000 pairs, n 6 l 5)
-    const int64_t slots = groups == 2 ? 8 : 16;
+    const int64_t slots = poly_group_slots(groups);
     const int64_t tiles = ((std::max<int64_t>(1, g.row_bound) / slots + d.S) * slots + 15) / 16;
     a.split = static_cast<int>((tiles + kWaves - 1) / kWaves);
     a.share = tiles == 1 ? kWaves : tiles == 2 ? 2 : 1;

@@ -10,6 +10,7 @@ weights and every compression.  Gates as in test_gpu_parity.py: float64
 
 from __future__ import annotations
 
+import ctypes
 from types import SimpleNamespace
 
 import numpy as np
@@ -134,3 +135,61 @@ def test_polynomial_basis(hip_context, oracle, shape, average, name):
         assert np.all(np.isfinite(values))
         error = scaled_error(values, expected)
         assert error <= GATES[dtype], f"{shape} {average} {dtype} {name}: scaled error {error:.3e}"
+
+
+@pytest.mark.parametrize("l_max", [1, 10, 4])
+@pytest.mark.parametrize("average", ["off", "inner", "outer"])
+def test_polynomial_rows_past_a_slot(hip_context, oracle, l_max, average):
+    """Centres of more rows than the first slots hold (512; about 600 here):
+    the search is run again and its rows counted, so the slots' stride passes
+    the row bound that sizes the radial functions.  A host call, a resident
+    run, two pipelined frames and a no-allocation run, each against the
+    oracle; l_max 1 and 10 by row, 4 in step groups."""
+
+    rng = np.random.default_rng(l_max)
+    sizes, species, r_cut = (30, 24), SPECIES[:2], 7.6
+    positions, cells = [], []
+    for atoms in sizes:
+        edge = (atoms / 0.1) ** (1.0 / 3.0)
+        sites = np.stack(np.unravel_index(rng.permutation(64)[:atoms], (4, 4, 4)), axis=1)
+        positions.append((sites + 0.5) * edge / 4 + rng.uniform(-0.2, 0.2, (atoms, 3)))
+        cells.append(np.eye(3) * edge)
+    batch = SimpleNamespace(numbers=np.resize(species, sum(sizes)).astype(np.int32), positions=np.concatenate(positions),
+                            cells=np.asarray(cells), pbc=np.ones((2, 3), np.int32),
+                            offsets=np.concatenate([[0], np.cumsum(sizes)]))
+    arguments = dict(species=species, n_max=3, l_max=l_max, r_cut=r_cut, sigma=1.0, alphas=None, betas=None,
+                     average=average, options={"polynomial": basis_polynomial(r_cut, 3)})
+    expected = oracle.soap(batch, **arguments)
+    context = _hip.Context(0)  # whose slots no earlier batch has widened
+    plan = _hip.SoapPlan(context, dtype="float64", **arguments)
+    pitch = plan.features * 8
+    resident = _hip.DeviceBatch(plan, batch)
+    out = _hip.DeviceMemory(expected.nbytes)
+
+    def check(values, what):
+        error = scaled_error(values, expected)
+        assert error <= GATES["float64"], f"l_max {l_max} {average} {what}: scaled error {error:.3e}"
+
+    def rows():
+        return out.to_host(np.empty_like(expected))
+
+    try:
+        values, timing = plan.compute(batch)
+        assert timing["pairs"] > 512 * sum(sizes)
+        check(values, "compute")
+        resident.run(out.address, pitch)
+        check(rows(), "run")
+        resident.close()
+        resident = _hip.DeviceBatch(plan, batch)
+        for _ in range(2):
+            resident.run_frame(batch.positions, out.address, pitch)
+        resident.wait()
+        check(rows(), "frames")
+        context.check(context.lib.mdx_hip_soap_run_noalloc(context.handle, plan.handle, resident.handle,
+                                                           ctypes.c_void_p(out.address), pitch, None, None))
+        check(rows(), "noalloc")
+    finally:
+        out.free()
+        resident.close()
+        plan.close()
+        context.close()

@@ -19,7 +19,7 @@ import pytest
 
 from conftest import ROOT
 from mdescriptor_amd import _hip, workloads
-from mdescriptor_amd.descriptors.basis import basis_gto
+from mdescriptor_amd.descriptors.basis import basis_gto, basis_polynomial
 
 pytestmark = pytest.mark.gpu
 
@@ -231,5 +231,34 @@ def test_noalloc_weighted_plan_matches_device_run(context, average):
             rows, timing = _run(context, plan, batch, "mdx_hip_soap_run_noalloc")
             np.testing.assert_array_equal(rows, expected)
             assert timing.expansion_tiles == reference.expansion_tiles <= -1000
+    finally:
+        plan.close()
+
+
+@pytest.mark.parametrize("n_max,l_max", [(4, 1), (3, 10), (4, 4)])
+@pytest.mark.parametrize("average", ["off", "inner"])
+def test_noalloc_polynomial_plan_matches_device_run(context, n_max, l_max, average):
+    """The polynomial basis: its radial functions share the static array with
+    the graph, whose rows are counted before the expansion here, so a centre's
+    slots (512) are wider than its rows (about 230).  By row (l_max 1 and 10)
+    and in step groups."""
+
+    rng = np.random.default_rng(l_max)
+    atoms, edge = 2500, 29.24
+    sites = np.stack(np.unravel_index(rng.permutation(14 ** 3)[:atoms], (14,) * 3), axis=1)
+    positions = (sites + 0.5) * edge / 14 + rng.uniform(-0.3, 0.3, (atoms, 3))
+    batch = SimpleNamespace(numbers=np.where(np.arange(atoms) % 3 == 0, 8, 1).astype(np.int32), positions=positions,
+                            cells=np.eye(3)[None] * edge, pbc=np.ones((1, 3), np.int32),
+                            offsets=np.array([0, atoms], np.int64))
+    plan = _hip.SoapPlan(context, species=[1, 8], n_max=n_max, l_max=l_max, r_cut=4.5, sigma=1.0, alphas=None,
+                         betas=None, average=average, dtype="float64",
+                         options={"polynomial": basis_polynomial(4.5, n_max)})
+    try:
+        print(f"polynomial n {n_max} l {l_max} {average}", flush=True)
+        expected, reference = _run(context, plan, batch, "mdx_hip_soap_run")
+        assert 200 * atoms < reference.pairs < 400 * atoms
+        rows, timing = _run(context, plan, batch, "mdx_hip_soap_run_noalloc")
+        assert timing.expansion_tiles == reference.expansion_tiles
+        np.testing.assert_array_equal(rows, expected)
     finally:
         plan.close()
