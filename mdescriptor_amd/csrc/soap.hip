@@ -543,6 +543,19 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     d.C = p.coeff_size;
     const int64_t rows = p.average != 0 ? pb.structures : pb.atoms;
     if (rows == 0 || d.F == 0) return;
+    if (pb.atoms == 0) {
+        // averages over structures without atoms are zero rows: no graph, no
+        // row weights, no radial functions for an expansion to read
+        if (events != nullptr) MDX_HIP(hipEventRecord(events[2], stream));
+        launch_block_zero_rows(stream, pb.d_offsets.as<int64_t>(), pb.structures, out_device, pitch_bytes,
+                               p.features * p.out_dtype);
+        if (events != nullptr) {
+            MDX_HIP(hipEventRecord(events[3], stream));
+            MDX_HIP(hipEventRecord(events[4], stream));
+        }
+        if (timing != nullptr) timing->expansion_launches = timing->expansion_tiles = 0;
+        return;
+    }
 
     const int64_t budget = partial_budget(pb, g, p.weighted != 0);
     Choice choice = choose(p, pb, g, budget, 0);
@@ -809,6 +822,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                 // without weights every species weight is 1
                 ba.row_w = p.weighted != 0 ? d_row_w : p.d_species_w.as<double>();
                 ba.row_w_mask = p.weighted != 0 ? -1 : 0;
+                ba.polynomial = p.radial_basis == 1 ? 1 : 0;
                 ba.poly_g = d_poly;
                 ba.poly_first = md.poly_first;
                 ba.poly_groups = layout.groups;

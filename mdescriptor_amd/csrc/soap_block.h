@@ -77,6 +77,7 @@ struct BlockArgs {
     // polynomial basis: radial functions of the slice's pairs, a step group
     // of 64 values per degree and exp register at
     // [(centre - poly_first) * poly_groups + group][l][register][lane]
+    int polynomial; // that basis (poly_g set)
     const double* poly_g;
     int64_t poly_first, poly_groups;
     int summed;                          // mu1nu1: spectrum against the species-summed coefficients

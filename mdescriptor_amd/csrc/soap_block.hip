@@ -210,7 +210,7 @@ void launch_block_expand(hipStream_t stream, int l_max, int kg, int ncr, const B
         throw Error(MDX_INTERNAL, "outer average row does not fit the register-coefficient kernel's LDS");
     }
     if (a.out_bytes > a.table_dtype || a.row_w == nullptr ||
-        (a.poly_g != nullptr && (kg > kBlockPolyGroups || a.table_dtype != 8 || a.small_structures || a.outer_lds != 0))) {
+        (a.polynomial != 0 && (a.poly_g == nullptr || kg > kBlockPolyGroups || a.table_dtype != 8 || a.small_structures || a.outer_lds != 0))) {
         throw Error(MDX_INTERNAL, "register-coefficient kernel launched with inconsistent arguments");
     }
     e->launch(stream, a, count);

@@ -1191,7 +1191,7 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
     using Plain = std::integral_constant<int, kBlockPlain>;
     using Weighted = std::integral_constant<int, kBlockWeighted>;
     using Polynomial = std::integral_constant<int, kBlockPolynomial>;
-    if (a.poly_g != nullptr) {
+    if (a.polynomial != 0) {
         if constexpr (KG <= kBlockPolyGroups) {
             if (a.struct_offsets == nullptr) launch(F64{}, Rows{}, Polynomial{}); else launch(F64{}, Inner{}, Polynomial{});
         }

@@ -206,3 +206,48 @@ def test_outer_average_in_lds_on_register_coefficient_kernel(hip_context, oracle
     assert np.all(values[1] == 0)
     error = scaled_error(values, expected)
     assert error <= (F64_GATE if dtype == "float64" else F32_GATE), f"{case} {name} {dtype}: scaled error {error:.3e}"
+
+
+@pytest.mark.parametrize("name", ["default", "pow_w0", "polynomial", "polynomial_pow_w0", "mu1nu1"])
+@pytest.mark.parametrize("average", ["inner", "outer"])
+@pytest.mark.parametrize("atoms", [0, 3])
+def test_average_of_structures_without_atoms(hip_context, oracle, name, average, atoms):
+    """Zero rows, with and without a structure of `atoms` atoms between them:
+    in such a batch there may be no pair rows to weight or to expand."""
+
+    from types import SimpleNamespace
+
+    from mdescriptor_amd.descriptors.basis import basis_polynomial
+
+    options = {}
+    if "pow_w0" in name:
+        options = dict(option_arguments("pow_w0", [1, 8], 4.0, 3))
+    if "polynomial" in name:
+        options["polynomial"] = basis_polynomial(4.0, 3)
+    if name == "mu1nu1":
+        options["compression"] = name
+    batch = SimpleNamespace(numbers=np.array([8, 1, 1], np.int32)[:atoms],
+                            positions=np.array([[0.0, 0, 0], [0.9, 0.1, 0], [-0.2, 0.9, 0.3]])[:atoms],
+                            cells=np.zeros((4, 3, 3)), pbc=np.zeros((4, 3), np.int32),
+                            offsets=np.array([0, 0, atoms, atoms, atoms]))
+    alphas, betas = basis_gto(4.0, 3, 4) if "polynomial" not in options else (None, None)
+    arguments = dict(species=[1, 8], n_max=3, l_max=4, r_cut=4.0, sigma=1.0, alphas=alphas, betas=betas,
+                     average=average, options=options)
+    expected = oracle.soap(batch, **arguments)
+    assert np.all(expected[[0, 2, 3]] == 0)
+    plan = _hip.SoapPlan(hip_context, dtype="float64", **arguments)
+    resident = _hip.DeviceBatch(plan, batch)
+    out = _hip.DeviceMemory(expected.nbytes)
+    try:
+        values, timing = plan.compute(batch)
+        assert scaled_error(values, expected) <= F64_GATE
+        assert np.all(values[[0, 2, 3]] == 0)
+        resident.run_frame(batch.positions, out.address, plan.features * 8)
+        resident.wait()
+        np.testing.assert_array_equal(out.to_host(np.empty_like(expected)), values)
+        resident.run(out.address, plan.features * 8)
+        np.testing.assert_array_equal(out.to_host(np.empty_like(expected)), values)
+    finally:
+        out.free()
+        resident.close()
+        plan.close()
