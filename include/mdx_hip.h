@@ -209,13 +209,15 @@ int mdx_hip_soap_run(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, mdx_device_bat
 
 /* mdx_hip_soap_run without device allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory during the run
- * (tight serving loops, code that must not call hipMalloc).  Same arguments,
- * results as mdx_hip_soap_run; the run's scratch (neighbour graph,
- * partial sums of the averaged modes) lives in one static device array of
+ * (tight serving loops, code that must not call hipMalloc).  Same arguments
+ * and results as mdx_hip_soap_run; the run's scratch (neighbour graph, row
+ * weights, radial functions of the polynomial basis, partial sums of the
+ * averaged modes) lives in one static device array of
  * MDX_NOALLOC_SCRATCH_BYTES per device instead of buffers owned by the batch.
  * Averages whose partial rows do not fit beside the graph take longer runs of
- * centres, then a workgroup per structure or a kernel with smaller rows: the
- * same features up to rounding.
+ * centres, then a workgroup per structure or a kernel with smaller rows;
+ * weighted plans and the polynomial basis take a kernel that keeps no weights
+ * or radial functions in memory: the same features up to rounding.
  * The plan, the batch and out_device are the caller's, made beforehand.  A
  * batch whose scratch does not fit returns MDX_INVALID_ARGUMENT with a message
  * that names the maximum.  All contexts on one device share its array, which

@@ -718,6 +718,7 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
             md.compression = plan->compression;
             md.radial = plan->radial_basis;
             md.grid = plan->grid_size;
+            md.poly_inside = 1; // the wider of the two forms in LDS
             md.crow = mdx::mfma_coefficient_rows(plan->Sc, n, plan->compression);
             md.n = n;
             md.l_max = p.l_max;
@@ -735,7 +736,7 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
             plan->clamp = md.clamp;
             // the workgroup's LDS: 160 KiB on gfx950 (dynamic, no opt-in needed)
             const size_t lds_limit = mdx::device_workgroup_lds();
-            const bool fits = mdx::mfma_template_tiles(mp.tiles) > 0 && mdx::mfma_lds_bytes(md) + mdx::mfma_plan_reserve(md) <= lds_limit;
+            const bool fits = mdx::mfma_template_tiles(mp.tiles) > 0 && mdx::mfma_lds_bytes(md) <= lds_limit;
             // only the matrix-core kernel implements weighting, compression and the polynomial basis
             const bool defaults = plan->compression == 0 && plan->radial_basis == 0 && plan->weighted == 0;
             plan->use_mfma = fits && (choice != "generic" || !defaults);

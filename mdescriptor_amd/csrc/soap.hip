@@ -31,6 +31,15 @@ constexpr int kItemCentres = 32;
 // polynomial basis: bytes of radial functions a slice of centres holds, at
 // most (what the last-level cache keeps between the two kernels of a slice)
 constexpr int64_t kPolySliceBytes = int64_t(256) << 20;
+// ... and the fewest centres of a slice: with less room the 16x16 kernel forms
+// the functions itself (as fast as slices of 128 centres on the register-
+// coefficient kernel: 3,000 atoms, n 6 l 5, 1,255 us, in slices of 128, 256
+// and 1,024 centres 1,221, 840 and 507; n 3 l 2, 639 and 756, 522, 325).  By
+// row as many as give the device 2,048 wavefronts, one per centre and tile
+// (n 4 l 1, a tile: 662 us, in slices of 512, 1,024 and 3,000 centres 1,071,
+// 691 and 524; n 3 l 10, eight tiles: 5,751 us, of 256 centres 1,331)
+constexpr int64_t kPolyLeastCentres = 256, kPolyLeastWaves = 2048;
+constexpr size_t kPolySlack = 4096; // alignment of the scratch's parts
 constexpr int kFoldItems = 16;  // rows per split, at least
 constexpr int kFoldSplits = 32; // splits per structure, at most
 
@@ -422,14 +431,17 @@ struct Choice {
     bool block_outer = false;     // ... a float64 partial row per centre
     bool block_outer_lds = false; // ... a workgroup per structure, power spectra summed in LDS
     bool quad = false;            // the 4x4-block kernel
+    bool poly_inside = false;     // polynomial basis: radial functions in the 16x16 kernel, without scratch
     int64_t largest_structure = 0;
     int64_t run = kItemCentres;   // centres per run
     size_t partial_width = 0;     // doubles of a partial row
     bool partials() const { return !block_inner && !block_outer_lds; } // (of an average)
 };
 
-// saving: 0 what is fastest; 1 no more scratch than runs of kItemCentres
-// take; 2 without the register-coefficient kernel's partial rows
+// Scratch a run may save: kFastest, no more of it than runs of kItemCentres
+// take, none for the register-coefficient kernel's partial rows, none beside
+// the other kernels' partial rows (no row weights, no radial functions).
+constexpr int kFastest = 0, kLongRuns = 1, kShortRows = 2, kLeast = 3;
 Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g, int64_t budget, int saving) {
     Choice c;
     const double F = static_cast<double>(p.features);
@@ -455,7 +467,7 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
     const double centre_rows = static_cast<double>(pb.atoms + 5 * pb.structures) * F * 8.0;
     const bool few = pb.structures < 2 * units && centre_rows <= static_cast<double>(budget);
     const bool outer_lds = p.average == 2 && whole && p.radial_basis == 0 && F * sizeof(double) <= static_cast<double>(kBlockOuterLdsBytes) &&
-                           (!few || saving > 0);
+                           (!few || saving > kFastest);
     const bool outer_rows = static_cast<double>(pb.atoms) * F * 8.0 <= 4294967296.0;
     // Three radial groups pad the power spectrum's Gram tiles (a register per
     // species), which centres of few neighbours do not repay: 1,000 molecules
@@ -465,11 +477,14 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
     // species 833 and 655)
     const bool padded = p.block_kg == 3 && p.block_ncr >= (p.average == 2 ? 3 : 5) && p.average != 1 && p.use_mfma &&
                         !p.block_forced && pb.most_images <= kBlockSmallAtoms;
-    c.block = p.block_waves > 0 && (p.average != 2 || outer_rows || outer_lds) && !padded && g.row_bound < kQuadMaxRows;
+    const bool scratch_rows = p.weighted != 0 || p.radial_basis == 1;
+    c.block = p.block_waves > 0 && (p.average != 2 || outer_rows || outer_lds) && !padded && g.row_bound < kQuadMaxRows &&
+              !(saving == kLeast && scratch_rows && p.use_mfma && !p.block_forced);
+    c.poly_inside = saving == kLeast && p.radial_basis == 1 && !c.block;
     const size_t block_width = c.block ? static_cast<size_t>(block_partial_width(p.l_max, p.block_ncr)) : 0;
     // A few small periodic structures hold thousands of pairs each (a
     // workgroup takes about a microsecond per 32 of them): runs too.
-    const bool spread = saving == 0 && !p.block_forced && pb.structures < units &&
+    const bool spread = saving == kFastest && !p.block_forced && pb.structures < units &&
                         c.largest_structure * std::min(pb.most_images, g.row_bound) > kBlockSpreadPairs &&
                         static_cast<double>(pb.atoms + 5 * pb.structures) * static_cast<double>(block_width) * 8.0 <=
                             static_cast<double>(budget);
@@ -477,7 +492,7 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
     c.block_outer_lds = c.block && outer_lds;
     c.block_runs = c.block && p.average == 1 && !c.block_inner;
     c.block_outer = c.block && p.average == 2 && !outer_lds;
-    if (saving == 2 && (c.block_runs || c.block_outer) && !p.block_forced) {
+    if (saving >= kShortRows && (c.block_runs || c.block_outer) && !p.block_forced) {
         c.block = c.block_runs = c.block_outer = false;
     }
     // else the 4x4-block kernel where the plan chose it (its coefficient rows
@@ -489,7 +504,7 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
                       : p.use_mfma     ? static_cast<size_t>(rows) * static_cast<size_t>(p.hpad)
                                        : static_cast<size_t>(p.coeff_size);
     if (p.average != 0 && c.partials() && !c.block_outer) {
-        c.run = saving == 0 ? run_centres(pb, c.partial_width, budget) : kItemCentres;
+        c.run = saving == kFastest ? run_centres(pb, c.partial_width, budget) : kItemCentres;
     }
     return c;
 }
@@ -508,7 +523,23 @@ Fold fold_of(int64_t most_items) {
     return f;
 }
 
-// Scratch of a run: its partial rows, folded rows, item tables and row weights.
+// The polynomial basis' radial functions of a run.
+PolyLayout poly_layout_of(const mdx_soap_plan& p, const DeviceGraph& g, const Choice& c) {
+    if (p.radial_basis != 1 || c.poly_inside) return {};
+    return poly_layout(g.row_bound, p.S, p.L, p.n, c.block);
+}
+
+// The least scratch for them: a slice's centres, at least an item's.
+size_t poly_least_bytes(const mdx_soap_plan& p, const PreparedBatch& pb, const PolyLayout& layout, const Choice& c) {
+    if (layout.centre == 0) return 0;
+    const int64_t item = c.block_inner ? c.largest_structure : p.average != 0 && !c.block_outer ? c.run : 1;
+    const int64_t slice = c.block ? kPolyLeastCentres : std::max(kPolyLeastCentres, kPolyLeastWaves / p.tiles);
+    const int64_t centres = std::min(pb.atoms, std::max(item, slice));
+    return static_cast<size_t>(centres * layout.centre) * sizeof(double) + kPolySlack;
+}
+
+// Scratch of a run beside the radial functions: its partial rows, folded
+// rows, item tables and row weights.
 size_t scratch_bytes(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g, const Choice& c) {
     size_t bytes = c.block && p.weighted != 0 ? static_cast<size_t>(graph_rows(pb, g)) * sizeof(double) + 256 : 0;
     if (p.average == 0 || !c.partials()) return bytes;
@@ -558,11 +589,16 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     }
 
     const int64_t budget = partial_budget(pb, g, p.weighted != 0);
-    Choice choice = choose(p, pb, g, budget, 0);
+    Choice choice = choose(p, pb, g, budget, kFastest);
     if (partials.arena != nullptr) {
         // the static array of a no-allocation run: what does not fit there
-        // takes long runs, then the tile kernels' short partial rows
-        for (int saving = 1; saving <= 2 && scratch_bytes(p, pb, g, choice) > partials.arena->left() + partials.bytes; ++saving) {
+        // takes long runs, then the tile kernels' short partial rows, then
+        // those kernels without row weights or radial functions in memory
+        const size_t room = partials.arena->left() + partials.bytes;
+        auto fits = [&](const Choice& c) {
+            return scratch_bytes(p, pb, g, c) + poly_least_bytes(p, pb, poly_layout_of(p, g, c), c) <= room;
+        };
+        for (int saving = kLongRuns; saving <= kLeast && !fits(choice); ++saving) {
             choice = choose(p, pb, g, budget, saving);
         }
     }
@@ -617,13 +653,12 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     };
     int64_t poly_centres = 0;
     size_t poly_bytes = 0;
-    PolyLayout layout;
-    if (p.radial_basis == 1) {
-        layout = poly_layout(g.row_bound, p.S, p.L, p.n, block);
+    const PolyLayout layout = poly_layout_of(p, g, choice);
+    if (layout.centre > 0) {
         const int64_t centre_bytes = layout.centre * static_cast<int64_t>(sizeof(double));
         int64_t room = kPolySliceBytes;
         if (partials.arena != nullptr) {
-            const size_t left = partials.arena->left() + partials.bytes, used = scratch_bytes(p, pb, g, choice) + 4096;
+            const size_t left = partials.arena->left() + partials.bytes, used = scratch_bytes(p, pb, g, choice) + kPolySlack;
             room = std::min(room, static_cast<int64_t>(left > used ? left - used : 0));
         }
         poly_centres = room / centre_bytes;
@@ -738,6 +773,12 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         tab.fbase = p.d_fbase.as<int32_t>();
         tab.fstride = p.d_fstride.as<int32_t>();
         tab.species_w = p.d_species_w.as<double>();
+        md.poly_inside = choice.poly_inside ? 1 : 0;
+        if (p.radial_basis == 1) {
+            const PolyTables t = poly_tables(p.d_poly.as<double>(), p.grid_size, p.n);
+            tab.poly_points = t.points;
+            tab.poly_basis = t.basis;
+        }
         tab.poly_g = d_poly;
         tab.poly_centre = layout.centre;
         tab.bin_atom = g.bin_atom.as<int32_t>();
@@ -784,7 +825,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         for (int64_t base = 0; base < items; base += count) {
             if (cancel != nullptr && *cancel != 0) throw Error(MDX_CANCELLED, "descriptor computation was cancelled");
             count = std::min(slice, items - base);
-            if (p.radial_basis == 1) {
+            if (layout.centre > 0) {
                 // as many items as the radial functions have room for
                 const int64_t first = first_centre(base), most = count;
                 for (count = 1; count < most && first_centre(base + count + 1) - first <= poly_centres;) ++count;

@@ -28,6 +28,7 @@ struct MfmaDims {
     int radial;      // 0 GTO, 1 polynomial
     int grid;        // polynomial radial grid points
     int64_t poly_first; // polynomial: first centre of the slice poly_g holds
+    int poly_inside;    // polynomial: the radial functions in the expansion itself (no poly_g)
     int weighted;    // 1 when any neighbour weight can differ from 1
     int weighting;   // 0 none, 1 poly, 2 pow, 3 exp
     int has_w0;
@@ -54,6 +55,8 @@ struct MfmaTables {
     const int32_t* fbase;
     const int32_t* fstride;
     const double* species_w;  // species weights [S]
+    const double* poly_points; // polynomial, in the expansion itself: r_q and the weighted basis (PolyTables)
+    const double* poly_basis;
     const double* poly_g;     // polynomial: radial functions of the slice's pair rows (launch_poly_radial)
     int64_t poly_centre;      // polynomial: doubles a centre in poly_g (PolyLayout)
     const int32_t* bin_atom;  // atom of each binned image (exact-self test for w0)
@@ -132,11 +135,6 @@ void launch_quad_expand(hipStream_t stream, int waves, int kg, int instr, const 
 inline int mfma_coefficient_rows(int Sc, int n, int compression) { return Sc * n + (compression == 2 ? n : 0) + 1; }
 int mfma_padded_row(int l_max);
 size_t mfma_lds_bytes(const MfmaDims& d);
-// LDS a polynomial plan must leave free beside that (once the radial kernels
-// of a grid step): the limit on its shape
-inline size_t mfma_plan_reserve(const MfmaDims& d) {
-    return d.radial == 1 ? static_cast<size_t>(d.L) * 32 * 4 * sizeof(double) : 0;
-}
 void launch_mfma_expand(hipStream_t stream, int template_tiles, const PreparedBatch& pb, const DeviceGraph& g,
                         const MfmaTables& tab, const MfmaDims& d, const int64_t* item_begin, int64_t base,
                         int64_t count, void* out, int64_t pitch, double* partial);
@@ -153,7 +151,14 @@ void launch_mfma_finalize(hipStream_t stream, const PreparedBatch& pb, const Mfm
 // the weighted basis w_q r_q^2 g_k(r_q) at 4 poly_channel_groups(n) channels
 // a point, padded to whole steps of four points; then the rows of a pair at
 // distance zero).  bw is the weighted basis, [q * n + k].
-int poly_channel_groups(int n);
+__host__ __device__ inline int poly_channel_groups(int n) { return n <= 4 ? 1 : n <= 8 ? 2 : 4; }
+struct PolyTables {
+    const double *points, *inverse, *basis, *centre;
+};
+inline PolyTables poly_tables(const double* tables, int grid, int n) {
+    const int64_t padded = (grid + 3) / 4 * 4;
+    return {tables, tables + padded, tables + 2 * padded, tables + padded * (2 + 4 * poly_channel_groups(n))};
+}
 std::vector<double> poly_radial_tables(int grid, int n, double eta, const double* points, const std::vector<double>& bw);
 void launch_poly_radial(hipStream_t stream, const PreparedBatch& pb, const DeviceGraph& g, const double* tables,
                         const MfmaDims& d, int64_t first, int64_t count, const PolyLayout& layout, double* out,

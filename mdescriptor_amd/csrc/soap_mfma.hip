@@ -72,11 +72,218 @@ __device__ inline double neighbour_weight(const MfmaDims& d, double distance, bo
     return value * species_w;
 }
 
+// Radial functions of the polynomial basis for the chunk's slots:
+//   G[slot][l*n + k] = sum_q K_l(q; r_slot) w_q r_q^2 g_k(r_q),
+// K_l the Gaussian-smeared radial kernel of polynomial_flir
+// (soap.cpp:450-492) with its l = 0 special case at r <= 1e-14.  Four grid
+// points at a time: one thread per (slot, point) evaluates K_0..K_lmax into
+// s_f, then each (l, 16-slot tile) unit -- one wavefront's -- adds its
+// 16 slots x 4 points x n product, computed on the matrix cores, into s_g.
+// All threads take part (barriers inside).  This and the next function serve
+// no-allocation runs whose scratch has no room for a slice of radial
+// functions (launch_poly_radial): 3,000 atoms, n 6 l 5, 1,257 us against 503.
+__device__ void polynomial_radial(const double* s_r, double* s_f, double* s_g, const MfmaTables& tab,
+                                  const MfmaDims& d, int tid, int wave, int threads, int waves) {
+    const int lane = tid % kWaveThreads;
+    const int L = d.L, n = d.n, Q = d.grid;
+    const int GP = L * n + 1;
+    const int stride = 4 * poly_channel_groups(n);
+    constexpr int kF = kNb * 4;  // entries of one l in s_f
+    for (int i = tid; i < kNb * GP; i += threads) s_g[i] = 0.0;
+    for (int q0 = 0; q0 < Q; q0 += 4) {
+        // (a workgroup of one wavefront takes two items per thread)
+        for (int item = tid; item < kF; item += threads) {
+            const int slot = item / 4, qq = item - slot * 4, q = q0 + qq;
+            double* f = s_f + slot * 4 + qq;
+            if (q < Q) {
+                const double radius = s_r[slot];
+                const double radial = tab.poly_points[q];
+                const double eta = d.eta;
+                if (radius <= 1e-14) {
+                    const double radial2 = radial * radial;
+                    f[0] = exp(-eta * radial2);
+                    for (int l = 1; l < L; ++l) f[l * kF] = 0.0;
+                } else {
+                    const double prefactor = 0.25 / (eta * radius * radial);
+                    const double minus = exp(-eta * (radial - radius) * (radial - radius));
+                    const double plus = exp(-eta * (radial + radius) * (radial + radius));
+                    double before = prefactor * (minus - plus);
+                    f[0] = before;
+                    if (L > 1) {
+                        double last = prefactor * (minus + plus - 2.0 * before);
+                        f[kF] = last;
+                        for (int l = 2; l < L; ++l) {
+                            const double value = before - prefactor * (4.0 * l - 2.0) * last;
+                            const double kept = value > 0.0 ? value : 0.0;
+                            f[l * kF] = kept;
+                            before = last;
+                            last = kept;
+                        }
+                    }
+                }
+            } else {
+                for (int l = 0; l < L; ++l) f[l * kF] = 0.0;
+            }
+        }
+        __syncthreads();
+        for (int u = wave; u < 2 * L; u += waves) {
+            const int l = u >> 1, tile = u & 1;
+            const double a = s_f[l * kF + (16 * tile + lane % 16) * 4 + lane / 16];
+            const int q = q0 + lane / 16;
+            const double b = q < Q && lane % 16 < n ? tab.poly_basis[q * stride + lane % 16] : 0.0;
+            const d4 g = mfma(a, b, d4{0.0, 0.0, 0.0, 0.0});
+            if (lane % 16 < n) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s_g[(16 * tile + lane / 16 + 4 * r) * GP + l * n + lane % 16] += g[r];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// The same radial functions with the sums over the grid in registers: up
+// to kPolyDegrees degrees (L) and kPolyGroups radial groups, the common
+// case.  A wavefront takes one half
+// of the chunk's slots and one of P parts of the grid, four points at a
+// time.  Lane L evaluates K_0..K_{L-1} for slot L % 16 of its half at grid
+// point L / 16 of the four, which is the A operand of v_mfma_f64_4x4x4f64
+// (block b = (L / 4) % 4 holds slots 4b..4b+3: A_b lane L = A_b[slot
+// L % 4][point L / 16]); the B operand is the quadrature-weighted basis of
+// radial group g (B lane L = w_q r_q^2 g_{4g + L % 4}(r_q) at point L / 16,
+// the same for every block), so one MFMA per degree and radial group
+// accumulates 4 slots x 4 channels per block with no padded channels, and
+// no barrier sits inside the grid loop.  Result lane L holds slot
+// 4b + L / 16, channel 4g + L % 4.  The parts' results go to s_g in part
+// order (part 0 writes, the others add, a barrier between), so the sums do
+// not depend on the schedule.
+constexpr int kPolyDegrees = 8;
+constexpr int kPolyGroups = 2; // radial groups of 4 channels (n <= 8)
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+__device__ void polynomial_radial_regs(const double* s_r, double* s_g, const double* s_tab, const MfmaTables& tab,
+                                       const MfmaDims& d, int tid, int wave, int threads, int waves) {
+    const int lane = tid % kWaveThreads;
+    const int L = d.L, n = d.n, Q = d.grid;
+    const int KG = (n + 3) / 4;
+    const int GP = L * n + 1;
+    const int stride = 4 * poly_channel_groups(n);
+    const int parts = waves >= 2 ? waves / 2 : 1;
+    const int blocks = (Q + 3) / 4;                       // grid blocks of 4 points
+    const int per_part = (blocks + parts - 1) / parts;
+    const int units = waves >= 2 ? 2 * parts : 1;
+    const double eta = d.eta;
+    // the pad entry of every slot's row stays zero
+    for (int i = tid; i < kNb; i += threads) s_g[i * GP + GP - 1] = 0.0;
+    for (int u0 = 0; u0 < (waves >= 2 ? 1 : 2); ++u0) {
+        // one wavefront: both halves in turn; else unit = wavefront
+        const int unit = waves >= 2 ? wave : u0;
+        const bool active = unit < units || waves < 2;
+        const int half = waves >= 2 ? unit % 2 : u0;
+        const int part = waves >= 2 ? unit / 2 : 0;
+        double acc[kPolyDegrees][kPolyGroups];
+#pragma unroll
+        for (int l = 0; l < kPolyDegrees; ++l) {
+#pragma unroll
+            for (int g = 0; g < kPolyGroups; ++g) acc[l][g] = 0.0;
+        }
+        if (active) {
+            const double radius = s_r[16 * half + lane % 16];
+            const int b0 = part * per_part, b1 = min(blocks, b0 + per_part);
+            // two grid blocks per iteration: their table loads, exps and
+            // degree recurrences are independent, so their latencies overlap
+            for (int blk0 = b0; blk0 < b1; blk0 += 2) {
+                double a_before[2], a_last[2], a_pref[2], bb[2][kPolyGroups];
+                bool a_centre[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int blk = blk0 + u;
+                    const int q = 4 * blk + lane / 16;
+                    const bool on_grid = blk < b1 && q < Q;
+                    const double radial = on_grid ? tab.poly_points[q] : 1.0;
+#pragma unroll
+                    for (int g = 0; g < kPolyGroups; ++g) {
+                        const int k = 4 * g + lane % 4;
+                        bb[u][g] = g < KG && on_grid && k < n ? tab.poly_basis[q * stride + k] : 0.0;
+                    }
+                    // K_l (soap.cpp:450-492): the l = 0 special case at r <= 1e-14
+                    double before, last;
+                    const bool at_centre = radius <= 1e-14;
+                    double prefactor = 0.0;
+                    if (at_centre) {
+                        before = exp_neg(-eta * (radial * radial), s_tab);
+                        last = 0.0;
+                    } else {
+                        prefactor = 0.25 / (eta * radius * radial);
+                        const double minus = exp_neg(-eta * (radial - radius) * (radial - radius), s_tab);
+                        const double plus = exp_neg(-eta * (radial + radius) * (radial + radius), s_tab);
+                        before = prefactor * (minus - plus);
+                        last = prefactor * (minus + plus - 2.0 * before);
+                    }
+                    if (!on_grid) {
+                        before = 0.0;
+                        last = 0.0;
+                    }
+                    a_before[u] = before;
+                    a_last[u] = last;
+                    a_pref[u] = prefactor;
+                    a_centre[u] = at_centre;
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int g = 0; g < kPolyGroups; ++g) acc[0][g] = mfma4(a_before[u], bb[u][g], acc[0][g]);
+                }
+#pragma unroll
+                for (int l = 1; l < kPolyDegrees; ++l) {
+                    // every degree and radial group, without a branch: the
+                    // sums of degrees past L are never stored, and groups
+                    // past KG meet a zero basis
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        double value = a_last[u];
+                        if (l >= 2) {
+                            const double next = a_before[u] - a_pref[u] * (4.0 * l - 2.0) * a_last[u];
+                            value = a_centre[u] ? 0.0 : (next > 0.0 ? next : 0.0);
+                            a_before[u] = a_last[u];
+                            a_last[u] = value;
+                        }
+#pragma unroll
+                        for (int g = 0; g < kPolyGroups; ++g) acc[l][g] = mfma4(value, bb[u][g], acc[l][g]);
+                    }
+                }
+            }
+        }
+        // the parts' sums, in part order
+        const int slot = 16 * half + 4 * ((lane / 4) % 4) + lane / 16;
+        for (int p = 0; p < parts; ++p) {
+            if (active && part == p) {
+#pragma unroll
+                for (int l = 0; l < kPolyDegrees; ++l) {
+#pragma unroll
+                    for (int g = 0; g < kPolyGroups; ++g) {
+                        const int k = 4 * g + lane % 4;
+                        if (l < L && g < KG && k < n) {
+                            double& v = s_g[slot * GP + l * n + k];
+                            v = p == 0 ? acc[l][g] : v + acc[l][g];
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Where the polynomial basis' radial functions come from: the rows that
+// launch_poly_radial left, or the kernel itself.
+constexpr int kPolyNone = 0, kPolyRows = 1, kPolyInside = 2;
+
 // kGeneral adds neighbour weights (kPoly: and the polynomial basis, whose
-// radial functions launch_poly_radial leaves per pair row); without them the
+// sums over the grid hold registers of their own inside); without them the
 // kernel keeps at least 4 wavefronts per SIMD (a 128-VGPR budget the
 // compiler must fit), with them 2.
-template <int T, bool kGeneral, bool kPoly>
+template <int T, bool kGeneral, int kPoly>
 __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfma(
     const double* __restrict__ positions, const int64_t* __restrict__ pair_start, const int32_t* __restrict__ counts,
     const uint32_t* __restrict__ pair_bin, const double* __restrict__ bx, const double* __restrict__ by,
@@ -100,12 +307,13 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
     const int cw = d.crow * hp;           // c words, including the zero row
     const int GP = L * n + 1;             // polynomial radial row; entry L*n stays zero
     double* s_y = lds;                    // kNb * HP
-    double* s_d2 = s_y + kNb * HP;        // kNb: d^2 of the chunk's slots
+    double* s_d2 = s_y + kNb * HP;        // kNb: d^2 (kPolyInside: distance) of the chunk's slots
     double* s_tab = s_d2 + kNb;           // 64: 2^(j/64) for exp_neg
     double* s_c = s_tab + 64;             // cw (coefficients of the current centre, padded)
     double* s_csum = s_c + cw;            // cw (inner average only)
     double* s_g = s_csum + (d.mode == 1 ? cw : 0);     // polynomial: kNb * GP radial functions
-    int* s_loff = reinterpret_cast<int*>(s_g + (d.radial == 1 ? kNb * GP : 0)); // L + 1
+    double* s_f = s_g + (d.radial == 1 ? kNb * GP : 0); // kPolyInside: L * kNb * 4 radial kernels
+    int* s_loff = reinterpret_cast<int*>(s_f + (kPoly == kPolyInside ? L * kNb * 4 : 0)); // L + 1
     int* s_seg = s_loff + (L + 1);        // S + 1: first row of each species segment of the centre
     int* s_pseg = s_seg + (S + 1);        // S + 1: first slot of each segment (padded to 4)
     int* s_step = s_pseg + (S + 1);       // 1: species of the chunk's MFMA steps, 4 bits each
@@ -281,8 +489,8 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
                     if (kGeneral && d.weighted && prow >= 0) {
                         scale = neighbour_weight(d, sqrt(d2), pself, tab.species_w[pq]);
                     }
-                    double hx = dx, hy = dy, hz = dz;
-                    if (kPoly) {
+                    double hx = dx, hy = dy, hz = dz, slot_value = d2;
+                    if (kPoly != kPolyNone) {
                         // polynomial: harmonics of the direction, times 4 pi w (soap.cpp:833-836);
                         const double radius = sqrt(d2);
                         const double inverse = radius <= 1e-14 ? 0.0 : 1.0 / radius;
@@ -290,9 +498,10 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
                         hy = dy * inverse;
                         hz = dz * inverse;
                         scale *= 4.0 * kPi;
+                        if (kPoly == kPolyInside) slot_value = radius;
                     }
                     if (wave == 0) {
-                        if (comp == 0) s_d2[jj] = d2;
+                        if (comp == 0) s_d2[jj] = slot_value;
                         // coefficient species of the 8 MFMA steps, 4 bits each, from the
                         // lanes holding slots 0, 4, .., 28 (lanes 0, 8, .., 56); mu2
                         // sums every species into block 0
@@ -317,7 +526,7 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
                     asm volatile("" : "+v"(part));
                     harmonics_q(hx, hy, hz, scale, lm, mk, part, &kHarmonic + zero, s_y + jj * HP);
                 }
-                if constexpr (kPoly) {
+                if constexpr (kPoly == kPolyRows) {
                     // the radial functions of the chunk's rows (pad slots, whose
                     // harmonics are zero, and the pad entry: zero)
                     const double* rows = tab.poly_g + poly_row(tab.poly_centre, centre, d.poly_first, 0, L * n);
@@ -331,6 +540,13 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
                     }
                 }
                 __syncthreads();
+                if constexpr (kPoly == kPolyInside) {
+                    if (L <= kPolyDegrees && n <= 4 * kPolyGroups) {
+                        polynomial_radial_regs(s_d2, s_g, s_tab, tab, d, tid, wave, kThreads, T);
+                    } else {
+                        polynomial_radial(s_d2, s_f, s_g, tab, d, tid, wave, kThreads, T);
+                    }
+                }
                 {
                     // issue the loads of the next chunk now
                     prow = slot_row(j0 + kNb + lane / 2, pq);
@@ -353,7 +569,7 @@ __global__ __launch_bounds__(T * kWaveThreads, kGeneral ? 2 : 4) void k_soap_mfm
 #pragma unroll
                         for (int s = 0; s < 4; ++s) {
                             const int jj = 4 * (h + s) + lane / 16;
-                            av[s] = !kPoly ? exp_neg(-expo * s_d2[jj], s_tab) : s_g[jj * GP + gcol];
+                            av[s] = kPoly == kPolyNone ? exp_neg(-expo * s_d2[jj], s_tab) : s_g[jj * GP + gcol];
                             yv[s] = s_y[jj * HP + ycol];
                         }
 #pragma unroll
@@ -451,8 +667,10 @@ void launch(hipStream_t stream, unsigned grid, int64_t per_block, size_t lds, co
             const DeviceGraph& g, const MfmaTables& tab, const MfmaDims& d, const int64_t* item_begin, int64_t base,
             int64_t count, void* out, int64_t pitch, double* partial) {
     const bool general = d.weighted != 0 || d.radial != 0;
-    auto kernel = d.radial != 0 ? k_soap_mfma<T, true, true> : general ? k_soap_mfma<T, true, false>
-                                                                       : k_soap_mfma<T, false, false>;
+    auto kernel = d.radial != 0 && d.poly_inside != 0 ? k_soap_mfma<T, true, kPolyInside>
+                  : d.radial != 0                     ? k_soap_mfma<T, true, kPolyRows>
+                  : general                           ? k_soap_mfma<T, true, kPolyNone>
+                                                      : k_soap_mfma<T, false, kPolyNone>;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(T * kWaveThreads), lds, stream, pb.d_positions.as<double>(),
                        g.pair_start.as<int64_t>(), g.counts.as<int32_t>(), g.pair_bin.as<uint32_t>(), g.bin_x.as<double>(),
                        g.bin_y.as<double>(), g.bin_z.as<double>(), tab, tab.ps_pref, d, item_begin, base,
@@ -571,6 +789,7 @@ size_t mfma_lds_bytes(const MfmaDims& d) {
     size_t words = static_cast<size_t>(kNb) * ((d.H + 1) | 1) + kNb + 64 + cw;
     if (d.mode == 1) words += cw;
     if (d.radial == 1) words += static_cast<size_t>(kNb) * (d.L * d.n + 1);
+    if (d.radial == 1 && d.poly_inside != 0) words += static_cast<size_t>(d.L) * kNb * 4;
     return words * sizeof(double) + static_cast<size_t>(d.L + 1 + 2 * (d.S + 1) + 1) * sizeof(int);
 }
 

@@ -253,8 +253,6 @@ void launch_degrees(hipStream_t stream, unsigned grid, const PolyArgs& a) {
 
 } // namespace
 
-int poly_channel_groups(int n) { return n <= 4 ? 1 : n <= 8 ? 2 : 4; }
-
 std::vector<double> poly_radial_tables(int grid, int n, double eta, const double* points, const std::vector<double>& bw) {
     const int groups = poly_channel_groups(n);
     const size_t padded = static_cast<size_t>((grid + 3) / 4 * 4);
@@ -292,10 +290,11 @@ void launch_poly_radial(hipStream_t stream, const PreparedBatch& pb, const Devic
     a.bx = g.bin_x.as<double>();
     a.by = g.bin_y.as<double>();
     a.bz = g.bin_z.as<double>();
-    a.points = tables;
-    a.inverse = tables + padded;
-    a.basis = a.inverse + padded;
-    a.centre = a.basis + padded * 4 * groups;
+    const PolyTables t = poly_tables(tables, d.grid, d.n);
+    a.points = t.points;
+    a.inverse = t.inverse;
+    a.basis = t.basis;
+    a.centre = t.centre;
     a.eta = d.eta;
     a.S = d.S;
     a.L = d.L;

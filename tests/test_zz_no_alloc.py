@@ -262,3 +262,66 @@ def test_noalloc_polynomial_plan_matches_device_run(context, n_max, l_max, avera
         np.testing.assert_array_equal(rows, expected)
     finally:
         plan.close()
+
+
+def _cell(atoms: int, seed: int) -> SimpleNamespace:
+    """One periodic cell of two species at 0.1 atoms per cubic angstrom."""
+
+    rng = np.random.default_rng(seed)
+    edge = (atoms / 0.1) ** (1.0 / 3.0)
+    side = int(np.ceil(atoms ** (1.0 / 3.0)))
+    sites = np.stack(np.unravel_index(rng.permutation(side ** 3)[:atoms], (side,) * 3), axis=1)
+    return SimpleNamespace(numbers=np.where(np.arange(atoms) % 3 == 0, 8, 1).astype(np.int32),
+                           positions=(sites + 0.5) * edge / side + rng.uniform(-0.3, 0.3, (atoms, 3)),
+                           cells=np.eye(3)[None] * edge, pbc=np.ones((1, 3), np.int32),
+                           offsets=np.array([0, atoms], np.int64))
+
+
+def _molecules(structures: int, atoms: int, seed: int) -> SimpleNamespace:
+    rng = np.random.default_rng(seed)
+    sites = np.stack(np.unravel_index(np.arange(atoms), (3, 3, 3)), axis=1) * 1.5
+    total = structures * atoms
+    return SimpleNamespace(numbers=np.where(np.arange(total) % 3 == 0, 8, 1).astype(np.int32),
+                           positions=np.tile(sites, (structures, 1)) + rng.uniform(-0.2, 0.2, (total, 3)),
+                           cells=np.zeros((structures, 3, 3)), pbc=np.zeros((structures, 3), np.int32),
+                           offsets=np.arange(structures + 1, dtype=np.int64) * atoms)
+
+
+@pytest.mark.parametrize("name,average,batch,l_max", [
+    ("pow_w0", "off", ("cell", 13000), 5),
+    ("pow_w0", "inner", ("molecules", 8000), 5),
+    ("pow_w0", "outer", ("cell", 13000), 2),
+    ("polynomial", "off", ("cell", 17500), 4),   # step groups where there is room
+    ("polynomial", "inner", ("cell", 17500), 4),
+    ("polynomial", "off", ("cell", 17500), 1),   # by row where there is room
+    ("polynomial_pow_w0", "off", ("cell", 17500), 10),
+])
+def test_noalloc_without_room_for_row_weights_or_radial_functions(context, name, average, batch, l_max):
+    """A batch whose graph leaves too little of the array for the row weights
+    or for a slice of radial functions: the kernel that needs neither takes
+    it, and nothing is refused."""
+
+    from conftest import scaled_error
+    from test_oracle_vs_reference import option_arguments
+
+    kind, size = batch
+    batch = _cell(size, 3) if kind == "cell" else _molecules(size, 20, 3)
+    options = {}
+    if "pow_w0" in name:
+        options.update(option_arguments("pow_w0", [1, 8], 4.5, 3))
+    alphas, betas = basis_gto(4.5, 3, l_max)
+    if "polynomial" in name:
+        options["polynomial"] = basis_polynomial(4.5, 3)
+        alphas = betas = None
+    plan = _hip.SoapPlan(context, species=[1, 8], n_max=3, l_max=l_max, r_cut=4.5, sigma=1.0, alphas=alphas,
+                         betas=betas, average=average, dtype="float64", options=options)
+    try:
+        print(f"{name} {average} {kind} {size} l {l_max}", flush=True)
+        expected, reference = _run(context, plan, batch, "mdx_hip_soap_run")
+        rows, timing = _run(context, plan, batch, "mdx_hip_soap_run_noalloc")
+        assert timing.pairs == reference.pairs
+        assert timing.expansion_tiles >= 0  # the 16x16 kernel
+        assert (reference.expansion_tiles <= -1000) == (2 <= l_max <= 9)
+        assert scaled_error(rows, expected) <= 1e-10
+    finally:
+        plan.close()
