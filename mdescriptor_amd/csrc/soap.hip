@@ -480,7 +480,18 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
     const bool scratch_rows = p.weighted != 0 || p.radial_basis == 1;
     c.block = p.block_waves > 0 && (p.average != 2 || outer_rows || outer_lds) && !padded && g.row_bound < kQuadMaxRows &&
               !(saving == kLeast && scratch_rows && p.use_mfma && !p.block_forced);
-    c.poly_inside = saving == kLeast && p.radial_basis == 1 && !c.block;
+    // By row the radial functions come a species at a time, padded to tiles of
+    // 16 rows; the 16x16 kernel forms those of 32 rows at once.  It is the
+    // faster of the two for up to eight degrees and channels (past them it
+    // meets a barrier every four grid points: from memory 2.6-6 times as
+    // fast) with more than six species, or three to six that do not fill two
+    // tiles each.  l 1, n 4, from memory and inside: 4,000 condensed atoms of
+    // two, four, six, ten species 604 and 830 us, 674 and 825, 822 and 870, 953
+    // and 922; 2,000 molecules of 9-29 atoms of two, three, six species 753 and
+    // 958, 1,313 and 1,067, 1,709 and 1,384; l 2 n 6, 4,000 atoms of nine 1,276
+    // and 1,024.
+    const bool short_tiles = p.S > 6 || (p.S > 2 && std::min(pb.most_images, g.row_bound) < 32 * p.S);
+    c.poly_inside = p.radial_basis == 1 && !c.block && (saving == kLeast || (p.L <= 8 && p.n <= 8 && short_tiles));
     const size_t block_width = c.block ? static_cast<size_t>(block_partial_width(p.l_max, p.block_ncr)) : 0;
     // A few small periodic structures hold thousands of pairs each (a
     // workgroup takes about a microsecond per 32 of them): runs too.
