@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <limits>
 
 namespace mdx {
 
@@ -499,7 +500,16 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
                         c.largest_structure * std::min(pb.most_images, g.row_bound) > kBlockSpreadPairs &&
                         static_cast<double>(pb.atoms + 5 * pb.structures) * static_cast<double>(block_width) * 8.0 <=
                             static_cast<double>(budget);
-    c.block_inner = c.block && p.average == 1 && whole && !spread;
+    // Centres of the polynomial basis that a slice of radial functions holds.
+    // A structure formed in one workgroup needs all of its centres at once: one
+    // past that (12,000 atoms among 1,024 molecules: 1.2 GB at l 2) sums runs,
+    // and no run is longer.
+    const PolyLayout poly = poly_layout(g.row_bound, p.S, p.L, p.n, c.block);
+    const int64_t slice_centres =
+        p.radial_basis != 1 || c.poly_inside
+            ? std::numeric_limits<int64_t>::max()
+            : std::max<int64_t>(1, kPolySliceBytes / (poly.centre * static_cast<int64_t>(sizeof(double))));
+    c.block_inner = c.block && p.average == 1 && whole && !spread && c.largest_structure <= slice_centres;
     c.block_outer_lds = c.block && outer_lds;
     c.block_runs = c.block && p.average == 1 && !c.block_inner;
     c.block_outer = c.block && p.average == 2 && !outer_lds;
@@ -515,7 +525,7 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
                       : p.use_mfma     ? static_cast<size_t>(rows) * static_cast<size_t>(p.hpad)
                                        : static_cast<size_t>(p.coeff_size);
     if (p.average != 0 && c.partials() && !c.block_outer) {
-        c.run = saving == kFastest ? run_centres(pb, c.partial_width, budget) : kItemCentres;
+        c.run = std::min<int64_t>(slice_centres, saving == kFastest ? run_centres(pb, c.partial_width, budget) : kItemCentres);
     }
     return c;
 }

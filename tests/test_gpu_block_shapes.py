@@ -194,3 +194,50 @@ def test_polynomial_rows_past_a_slot(hip_context, oracle, l_max, average):
         resident.close()
         plan.close()
         context.close()
+
+
+def _free_device_bytes() -> int:
+    runtime = _hip.DeviceMemory.runtime()
+    runtime.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]
+    runtime.hipMemGetInfo.restype = ctypes.c_int
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert runtime.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return int(free.value)
+
+
+def test_polynomial_large_structure_among_many(hip_context):
+    """Inner averages of enough structures for a workgroup each, one of them
+    too large for a slice of radial functions (256 MiB): its centres are
+    summed in runs, and the run takes little more memory than such a slice.
+    Rows against those of the two kinds of structure by themselves."""
+
+    rng = np.random.default_rng(4)
+    atoms, lone = 12000, 1100
+    edge = (atoms / 0.1) ** (1.0 / 3.0)
+    sites = np.stack(np.unravel_index(rng.permutation(23 ** 3)[:atoms], (23,) * 3), axis=1)
+    large = SimpleNamespace(numbers=np.resize([1, 8], atoms).astype(np.int32),
+                            positions=(sites + 0.5) * edge / 23 + rng.uniform(-0.3, 0.3, (atoms, 3)),
+                            cells=np.eye(3)[None] * edge, pbc=np.ones((1, 3), np.int32), offsets=np.array([0, atoms]))
+    pairs = SimpleNamespace(numbers=np.resize([1, 8], 2 * lone).astype(np.int32),
+                            positions=rng.uniform(0.5, 1.5, (2 * lone, 3)) + np.resize([[0.0] * 3, [1.0] * 3], (2 * lone, 3)),
+                            cells=np.zeros((lone, 3, 3)), pbc=np.zeros((lone, 3), np.int32),
+                            offsets=np.arange(lone + 1) * 2)
+    both = SimpleNamespace(numbers=np.concatenate([pairs.numbers, large.numbers]),
+                           positions=np.concatenate([pairs.positions, large.positions]),
+                           cells=np.concatenate([pairs.cells, large.cells]), pbc=np.concatenate([pairs.pbc, large.pbc]),
+                           offsets=np.concatenate([pairs.offsets, pairs.offsets[-1] + large.offsets[1:]]))
+    plan = _hip.SoapPlan(hip_context, species=[1, 8], n_max=3, l_max=2, r_cut=4.5, sigma=1.0, alphas=None, betas=None,
+                         average="inner", dtype="float64", options={"polynomial": basis_polynomial(4.5, 3)})
+    expected = np.concatenate([plan.compute(pairs)[0], plan.compute(large)[0]])
+    batch = _hip.DeviceBatch(plan, both)
+    out = _hip.DeviceMemory(expected.nbytes)
+    try:
+        free = _free_device_bytes()
+        timing = batch.run(out.address, plan.features * 8)
+        assert free - _free_device_bytes() < 500 << 20
+        assert timing["expansion_tiles"] <= -1000
+        assert scaled_error(out.to_host(np.empty_like(expected)), expected) <= GATES["float64"]
+    finally:
+        out.free()
+        batch.close()
+        plan.close()
