@@ -766,18 +766,24 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
             // species) shape.  It keeps its coefficients in registers, so the
             // tile kernel's LDS limit does not apply to it
             if (quad_range && (choice == "auto" || choice == "block")) {
-                mdx::BlockPlanHost bp;
-                double beta_largest = 0.0;
-                for (int i = 0; plan->radial_basis == 0 && i < L * n * n; ++i) beta_largest = std::max(beta_largest, std::fabs(p.betas[i]));
-                if (mdx::block_plan_tables(plan->S, n, p.l_max, p.out_dtype, p.average, plan->compression,
-                                           plan->weighted != 0, plan->radial_basis == 1, beta_largest, beta, pref, expo, bp)) {
-                    plan->block_table_dtype = bp.table_dtype;
+                plan->block_float32 = mdx::block_float32_exps(plan->S, n, p.l_max, p.out_dtype, p.average, plan->compression,
+                                                              plan->weighted != 0, plan->radial_basis == 1);
+                // (weighted inner averages run with either exps)
+                const bool either = plan->block_float32 && p.average == 1 && plan->weighted != 0;
+                for (int f32 = 0; f32 < 2; ++f32) {
+                    if ((f32 != 0) != plan->block_float32 && !either) continue;
+                    mdx::BlockPlanHost bp;
+                    if (!mdx::block_plan_tables(plan->S, n, p.l_max, f32 != 0 ? 4 : 8, plan->compression,
+                                                plan->radial_basis == 1, beta, pref, expo, bp)) {
+                        plan->block_waves = 0;
+                        break;
+                    }
                     plan->block_waves = bp.waves;
                     plan->block_kg = bp.kg;
                     plan->block_ncr = bp.ncr;
-                    upload(plan->d_block_e1, bp.lane_e1);
+                    upload(plan->d_block_e1[f32], bp.lane_e1);
                     upload(plan->d_block_beta, bp.lane_beta);
-                    upload(plan->d_block_ps, bp.ps_offsets);
+                    upload(plan->d_block_ps[f32], bp.ps_offsets);
                 }
             }
             plan->block_forced = choice == "block";

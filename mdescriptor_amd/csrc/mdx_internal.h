@@ -507,9 +507,12 @@ struct mdx_soap_plan {
     // register-coefficient kernel (soap_block.hip), default options and
     // average "off" only: wavefronts (0: not used), radial groups,
     // coefficient registers, lane tables
-    int block_waves = 0, block_kg = 0, block_ncr = 0, block_table_dtype = 8;
+    int block_waves = 0, block_kg = 0, block_ncr = 0;
+    bool block_float32 = false; // float32 exps (block_float32_exps)
     bool block_forced = false; // MDX_HIP_SOAP_KERNEL=block: also for inner averages of few large structures
-    mdx::DeviceBuffer d_block_e1, d_block_beta, d_block_ps;
+    // exp constants and feature offsets with float64 [0] and float32 [1] exps,
+    // those the plan may run
+    mdx::DeviceBuffer d_block_e1[2], d_block_beta, d_block_ps[2];
     // options beyond the GTO / uncompressed / unweighted default (mdx_soap_options)
     int Sc = 0;              // coefficient species: 1 for mu2, else S
     int compression = 0;     // 0 off, 1 mu2, 2 mu1nu1, 3 crossover

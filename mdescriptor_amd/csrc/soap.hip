@@ -431,6 +431,7 @@ struct Choice {
     bool block_runs = false;      // ... runs of a structure's centres into partial coefficient rows
     bool block_outer = false;     // ... a float64 partial row per centre
     bool block_outer_lds = false; // ... a workgroup per structure, power spectra summed in LDS
+    bool f32_exps = false;        // ... with float32 exps
     bool quad = false;            // the 4x4-block kernel
     bool poly_inside = false;     // polynomial basis: radial functions in the 16x16 kernel, without scratch
     int64_t largest_structure = 0;
@@ -509,6 +510,9 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
         p.radial_basis != 1 || c.poly_inside
             ? std::numeric_limits<int64_t>::max()
             : std::max<int64_t>(1, kPolySliceBytes / (poly.centre * static_cast<int64_t>(sizeof(double))));
+    // (weighted inner averages: those of few large structures only, whose
+    // former kernel had them)
+    c.f32_exps = c.block && p.block_float32 && !(p.average == 1 && p.weighted != 0 && whole);
     c.block_inner = c.block && p.average == 1 && whole && !spread && c.largest_structure <= slice_centres;
     c.block_outer_lds = c.block && outer_lds;
     c.block_runs = c.block && p.average == 1 && !c.block_inner;
@@ -863,11 +867,11 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                 ba.bx = g.bin_x.as<double>();
                 ba.by = g.bin_y.as<double>();
                 ba.bz = g.bin_z.as<double>();
-                ba.lane_e1 = p.d_block_e1.as<double>();
+                ba.lane_e1 = p.d_block_e1[choice.f32_exps].as<double>();
                 ba.lane_beta = p.d_block_beta.as<double>();
-                ba.ps_offsets = p.d_block_ps.as<int32_t>();
+                ba.ps_offsets = p.d_block_ps[choice.f32_exps].as<int32_t>();
                 ba.S = p.S;
-                ba.table_dtype = p.block_table_dtype;
+                ba.table_dtype = choice.f32_exps ? 4 : 8;
                 ba.out_bytes = block_outer ? 8 : p.out_dtype;
                 ba.F = p.features;
                 ba.item_base = base;

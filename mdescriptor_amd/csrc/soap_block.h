@@ -26,11 +26,12 @@ namespace mdx {
 // (summed: each channel against the species-summed channels) as a branch at
 // the end of a row, the others through the plan's tables.
 constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuterLds = 3;
-// ... and forms: unweighted, weighted (the weights may be 1), and the
-// polynomial basis (weighted the same way): the radial functions come from
-// memory (launch_poly_radial) instead of exps, rows and inner averages only,
-// up to two radial groups (its normalisation fails past eight channels).
-constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2;
+// ... and forms: unweighted, weighted (the weights may be 1), the polynomial
+// basis (weighted the same way): the radial functions come from memory
+// (launch_poly_radial) instead of exps, rows and inner averages only, up to
+// two radial groups (its normalisation fails past eight channels); and
+// unweighted float32 rows of float64 tables.
+constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2, kBlockHalf = 3;
 constexpr int kBlockPolyGroups = 2;
 // largest row (features x 8 bytes) the outer mode accumulates in LDS
 constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;
@@ -52,7 +53,7 @@ struct BlockArgs {
     const double* lane_beta;    // [l][fold term][64]: beta^T operand of the lane
     const int32_t* ps_offsets;  // [tile pair][value][64]: (byte offset at l = 0) << 9 | feature stride per l
     int S;                      // species
-    int table_dtype;            // bytes per value the plan's tables are for: 4 (float32 exps and rows) or 8
+    int table_dtype;            // bytes per value the tables are for: 4 (float32 exps and rows) or 8
     int out_bytes;              // bytes per output value, 4 or 8 (tables for 4: 4)
     int64_t F;                  // features per row
     int64_t item_base, items, per_block; // centres, or structures when struct_offsets is set
@@ -106,16 +107,14 @@ struct BlockPlanHost {
     int kg = 0;      // radial groups of 4 channels
     int ncr = 0;     // coefficient registers per (l, column group)
     int waves = 0;   // wavefronts per workgroup
-    int table_dtype = 8;
     std::vector<double> lane_e1, lane_beta;
     std::vector<int32_t> ps_offsets; // packed feature offsets
 };
 
 // One compiled shape (soap_block_shape.hip): l_max, radial groups,
 // coefficient registers.  every_form: compiled with float32 and float64 exps
-// for rows and inner averages, weighted or not; else float32 exps serve
-// unweighted rows only, and float64 tables everything else, whatever the
-// output type.
+// for rows and inner averages, weighted or not; else float64 exps serve
+// every output type.
 struct BlockShape {
     int l_max, kg, ncr;
     bool every_form;
@@ -126,13 +125,21 @@ struct BlockShape {
 // Fills out and returns true when a compiled shape holds (S, n, l_max).
 // compression: 0 off, 1 mu2 (one coefficient species: the shape of S
 // species, the feature layout of one), 2 mu1nu1, 3 crossover (the feature
-// layouts of soap.cpp:948-1013).  average: 0 off, 1 inner, 2 outer; weighted:
-// neighbour weights; polynomial: that radial basis (float64 tables).
-// beta_largest is the largest |beta| entry; out.table_dtype the value size
-// the tables are built for.
-bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted, bool polynomial,
-                       double beta_largest, const std::vector<double>& beta_scaled,
-                       const std::vector<double>& pref, const std::vector<double>& expo, BlockPlanHost& out);
+// layouts of soap.cpp:948-1013).  polynomial: that radial basis (float64
+// tables).  table_dtype: the value size the tables are built for.
+bool block_plan_tables(int S, int n, int l_max, int table_dtype, int compression, bool polynomial,
+                       const std::vector<double>& beta_scaled, const std::vector<double>& pref,
+                       const std::vector<double>& expo, BlockPlanHost& out);
+// Whether a plan takes float32 exps (relative error 1.4e-13 against 5e-15):
+// float32 rows of the shapes compiled in every form, and their uncompressed
+// inner averages (weighted ones as runs of centres only, Choice::f32_exps).
+// There the beta fold does not lift the difference to the rows' own rounding:
+// against float64 rows rounded to float32 (2.0-2.9e-8 of the row), twelve
+// channels in 5 A (max |beta| 2.0e5) are 1.0e-10 of the row off, in 4 A
+// (6.8e5) 5.5e-10, eight in 2 A (2.0e6) 8e-11.  average: 0 off, 1 inner, 2
+// outer (whose rows are float64 sums).
+bool block_float32_exps(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted,
+                        bool polynomial);
 void launch_block_expand(hipStream_t stream, int l_max, int kg, int ncr, const BlockArgs& a, int64_t count);
 // doubles in one partial row of the runs' launch
 int64_t block_partial_width(int l_max, int ncr);

@@ -33,9 +33,6 @@ const BlockShape* find_shape(int l_max, int kg, int ncr) {
     return best;
 }
 
-// largest |beta| of a basis whose float32 rows take the float32 exps
-constexpr double kFloat32ExpBeta = 2e4;
-
 int coefficient_registers(int S, int kg) { return kg == 3 ? S : (S * kg + 3) / 4; }
 
 } // namespace
@@ -44,9 +41,17 @@ int64_t block_partial_width(int l_max, int ncr) {
     return static_cast<int64_t>(units_total(0xffffffffu, l_max + 1)) * ncr * kWaveThreads;
 }
 
-bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted, bool polynomial,
-                       double beta_largest, const std::vector<double>& beta_scaled,
-                       const std::vector<double>& pref, const std::vector<double>& expo, BlockPlanHost& out) {
+bool block_float32_exps(int S, int n, int l_max, int out_dtype, int average, int compression, bool weighted,
+                        bool polynomial) {
+    const int kg = (n + 3) / 4;
+    const BlockShape* e = find_shape(l_max, kg, coefficient_registers(compression == 1 ? 1 : S, kg));
+    if (e == nullptr || !e->every_form || out_dtype != 4 || polynomial) return false;
+    return average == 0 ? compression != 2 || !weighted : average == 1 && compression == 0;
+}
+
+bool block_plan_tables(int S, int n, int l_max, int table_dtype, int compression, bool polynomial,
+                       const std::vector<double>& beta_scaled, const std::vector<double>& pref,
+                       const std::vector<double>& expo, BlockPlanHost& out) {
     out = BlockPlanHost{};
     if (compression < 0 || compression > 3) return false;
     // species of the coefficients and the feature layout (mu2: one)
@@ -57,15 +62,6 @@ bool block_plan_tables(int S, int n, int l_max, int out_dtype, int average, int 
     if (e == nullptr) return false;
     // registers past the species' stay zero, and no feature is stored from them
     const int ncr = e->ncr;
-    // An outer average sums float64 rows.  Float32 rows take the float32 exps
-    // (relative error 1.4e-13 more) where the beta fold cannot lift that to
-    // the rows' own rounding: max |beta| up to 2e4 (ten channels in 5 A have
-    // 1.3e4), or the shapes measured with it (twelve channels in 5.5 A, 1.2e5:
-    // rows 2.7e-8 off the exact values against 2.5e-8 of rounding)
-    const bool f32_exps =
-        !polynomial && e->every_form ? average != 2 : !polynomial && average == 0 && !weighted && beta_largest <= kFloat32ExpBeta;
-    const int table_dtype = f32_exps ? out_dtype : 8;
-    out.table_dtype = table_dtype;
     const int L = l_max + 1;
     {
         const int64_t W = static_cast<int64_t>(St) * n;
@@ -209,7 +205,7 @@ void launch_block_expand(hipStream_t stream, int l_max, int kg, int ncr, const B
                              a.F * static_cast<int64_t>(sizeof(double)) > kBlockOuterLdsBytes)) {
         throw Error(MDX_INTERNAL, "outer average row does not fit the register-coefficient kernel's LDS");
     }
-    if (a.out_bytes > a.table_dtype || a.row_w == nullptr ||
+    if (a.out_bytes > a.table_dtype || a.row_w == nullptr || (a.table_dtype == 4 && !e->every_form) ||
         (a.polynomial != 0 && (a.poly_g == nullptr || kg > kBlockPolyGroups || a.table_dtype != 8 || a.small_structures || a.outer_lds != 0))) {
         throw Error(MDX_INTERNAL, "register-coefficient kernel launched with inconsistent arguments");
     }

@@ -436,7 +436,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     // centres the same way, into a partial row)
     constexpr bool inner = MODE != kBlockRows;
     constexpr bool kPoly = FORM == kBlockPolynomial;
-    constexpr bool kWeighted = FORM != kBlockPlain;
+    constexpr bool kWeighted = FORM == kBlockWeighted || FORM == kBlockPolynomial;
     // outer averages in LDS: a structure's centres one by one, each centre's
     // power spectrum added into s_acc (F float64 values), its mean written
     // when the structure ends
@@ -699,10 +699,9 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     };
 
     const int64_t F = a.F;
-    // float32 rows of a plan whose tables are those of float64 rows (never the
-    // unweighted form, which is compiled with float32 tables too: the choice
-    // per store cost its float64 rows 1-2 %)
-    const bool half_rows = ES == 8 && FORM != kBlockPlain && a.out_bytes == 4;
+    // float32 rows of float64 tables (the unweighted forms decide at compile
+    // time: the choice per store cost float64 rows 1-2 %)
+    const bool half_rows = ES == 8 && (FORM == kBlockHalf || (kWeighted && a.out_bytes == 4));
     // row end: C <- (S_lm C)^T beta^T scaled by scale0, the power spectrum of
     // the owned degrees to output row row0, and C back to zero
     auto row_end = [&](int64_t row0, double scale0) {
@@ -1191,6 +1190,7 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
     using Plain = std::integral_constant<int, kBlockPlain>;
     using Weighted = std::integral_constant<int, kBlockWeighted>;
     using Polynomial = std::integral_constant<int, kBlockPolynomial>;
+    using Half = std::integral_constant<int, kBlockHalf>;
     if (a.polynomial != 0) {
         if constexpr (KG <= kBlockPolyGroups) {
             if (a.struct_offsets == nullptr) launch(F64{}, Rows{}, Polynomial{}); else launch(F64{}, Inner{}, Polynomial{});
@@ -1205,7 +1205,7 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
             if (f32) {
                 if (weighted) launch(F32{}, m, Weighted{}); else launch(F32{}, m, Plain{});
             } else {
-                if (weighted) launch(F64{}, m, Weighted{}); else launch(F64{}, m, Plain{});
+                if (weighted || a.out_bytes == 4) launch(F64{}, m, Weighted{}); else launch(F64{}, m, Plain{});
             }
         };
         if (outer) {
@@ -1213,14 +1213,17 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
         } else if (a.struct_offsets == nullptr) {
             typed(Rows{});
         } else if (a.small_structures) {
-            typed(Small{});
+            // (weighted: float64 exps)
+            if (f32) launch(F32{}, Small{}, Plain{});
+            else if (weighted || a.out_bytes == 4) launch(F64{}, Small{}, Weighted{});
+            else launch(F64{}, Small{}, Plain{});
         } else {
             typed(Inner{});
         }
     } else if (outer) {
         launch(F64{}, Outer{}, Weighted{});
     } else if (a.struct_offsets == nullptr) {
-        if (f32) launch(F32{}, Rows{}, Plain{}); else launch(F64{}, Rows{}, Weighted{});
+        if (a.out_bytes == 4 && !weighted) launch(F64{}, Rows{}, Half{}); else launch(F64{}, Rows{}, Weighted{});
     } else if (a.small_structures) {
         launch(F64{}, Small{}, Weighted{});
     } else {

@@ -12,7 +12,7 @@ namespace {
 
 // Shapes compiled in every form (float32 and float64 exps, with and without
 // neighbour weights): the sizes this package's workloads use.  The others have
-// five forms: unweighted float32 rows, and with float64 exps and weights that
+// float64 exps and five forms: unweighted float32 rows, and with weights that
 // may be 1 (2-4 % slower than a form without them) rows, inner averages, inner
 // averages of small structures and outer averages.
 constexpr bool every_form(int lm, int kg, int ncr) {

@@ -241,3 +241,38 @@ def test_polynomial_large_structure_among_many(hip_context):
         out.free()
         batch.close()
         plan.close()
+
+
+@pytest.mark.parametrize("shape,average,name", [
+    ((4, 4, 2), "off", "default"), ((3, 8, 7), "off", "default"), ((2, 5, 5), "off", "mu1nu1"),
+    ((2, 9, 5), "off", "default"), ((2, 9, 5), "off", "pow_w0"), ((3, 8, 7), "inner", "default"),
+    ((4, 7, 3), "outer", "default"),
+    # shapes whose float32 rows take float32 exps: not with these
+    ((4, 8, 6), "inner", "mu2"), ((4, 8, 6), "inner", "mu1nu1"), ((4, 8, 6), "inner", "pow_w0"),
+    ((4, 8, 6), "off", "pow_w0_mu1nu1"), ((5, 6, 4), "outer", "crossover"),
+])
+def test_float32_rows_of_float64_exps(hip_context, shape, average, name):
+    """Float32 rows that take the exps of float64 rows are those rows rounded,
+    bit for bit (exps of another error differ in some of them: a packed basis,
+    whose fold amplifies it).  Structures of at most a wavefront of atoms and
+    one past it."""
+
+    options = dict(POW_W0) if "pow_w0" in name else {}
+    if name.split("_")[-1] in ("mu2", "mu1nu1", "crossover"):
+        options["compression"] = name.split("_")[-1]
+    count, n_max, l_max = shape
+    r_cut = 4.0 if n_max > 8 else 3.0
+    alphas, betas = basis_gto(r_cut, n_max, l_max)
+    rows = {}
+    for sizes in ((21, 13, 1, 20), (70, 66)):
+        for dtype in ("float64", "float32"):
+            plan = _hip.SoapPlan(hip_context, species=SPECIES[:count], n_max=n_max, l_max=l_max, r_cut=r_cut, sigma=1.0,
+                                 alphas=alphas, betas=betas, average=average, dtype=dtype, options=options)
+            try:
+                rows[dtype], timing = plan.compute(_structures(sum(shape), sizes, SPECIES[:count]))
+            finally:
+                plan.close()
+            assert timing["expansion_tiles"] <= -1000
+        if average == "inner" and name == "pow_w0" and sizes[0] > 64:
+            continue  # a few large structures: float32 exps
+        np.testing.assert_array_equal(rows["float32"], rows["float64"].astype(np.float32))
