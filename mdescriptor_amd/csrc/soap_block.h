@@ -29,9 +29,10 @@ constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuter
 // ... and forms: unweighted, weighted (the weights may be 1), the polynomial
 // basis (weighted the same way): the radial functions come from memory
 // (launch_poly_radial) instead of exps, rows and inner averages only, up to
-// two radial groups (its normalisation fails past eight channels); and
-// unweighted float32 rows of float64 tables.
-constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2, kBlockHalf = 3;
+// two radial groups (its normalisation fails past eight channels);
+// unweighted float32 rows of float64 tables; and weighted rows of the tables'
+// own type (shapes compiled in every form).
+constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2, kBlockHalf = 3, kBlockWeightedRows = 4;
 constexpr int kBlockPolyGroups = 2;
 // largest row (features x 8 bytes) the outer mode accumulates in LDS
 constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;

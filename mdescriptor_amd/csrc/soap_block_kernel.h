@@ -436,7 +436,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     // centres the same way, into a partial row)
     constexpr bool inner = MODE != kBlockRows;
     constexpr bool kPoly = FORM == kBlockPolynomial;
-    constexpr bool kWeighted = FORM == kBlockWeighted || FORM == kBlockPolynomial;
+    constexpr bool kWeighted = FORM != kBlockPlain && FORM != kBlockHalf;
     // outer averages in LDS: a structure's centres one by one, each centre's
     // power spectrum added into s_acc (F float64 values), its mean written
     // when the structure ends
@@ -699,9 +699,11 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     };
 
     const int64_t F = a.F;
-    // float32 rows of float64 tables (the unweighted forms decide at compile
-    // time: the choice per store cost float64 rows 1-2 %)
-    const bool half_rows = ES == 8 && (FORM == kBlockHalf || (kWeighted && a.out_bytes == 4));
+    // float32 rows of float64 tables (three forms decide at compile time: the
+    // choice per store cost float64 rows 1-2 %, weighted ones 4-6 %: 1,000
+    // molecules of five species n 8 l 8, crossover, 366 and 401 us)
+    const bool half_rows =
+        ES == 8 && (FORM == kBlockHalf || (kWeighted && FORM != kBlockWeightedRows && a.out_bytes == 4));
     // row end: C <- (S_lm C)^T beta^T scaled by scale0, the power spectrum of
     // the owned degrees to output row row0, and C back to zero
     auto row_end = [&](int64_t row0, double scale0) {
@@ -1191,6 +1193,7 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
     using Weighted = std::integral_constant<int, kBlockWeighted>;
     using Polynomial = std::integral_constant<int, kBlockPolynomial>;
     using Half = std::integral_constant<int, kBlockHalf>;
+    using WeightedRows = std::integral_constant<int, kBlockWeightedRows>;
     if (a.polynomial != 0) {
         if constexpr (KG <= kBlockPolyGroups) {
             if (a.struct_offsets == nullptr) launch(F64{}, Rows{}, Polynomial{}); else launch(F64{}, Inner{}, Polynomial{});
@@ -1211,7 +1214,15 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
         if (outer) {
             if (weighted) launch(F64{}, Outer{}, Weighted{}); else launch(F64{}, Outer{}, Plain{});
         } else if (a.struct_offsets == nullptr) {
-            typed(Rows{});
+            if (weighted && a.out_bytes == a.table_dtype) {
+                if (f32) launch(F32{}, Rows{}, WeightedRows{}); else launch(F64{}, Rows{}, WeightedRows{});
+            } else if (f32) {
+                launch(F32{}, Rows{}, Plain{});
+            } else if (weighted || a.out_bytes == 4) {
+                launch(F64{}, Rows{}, Weighted{});
+            } else {
+                launch(F64{}, Rows{}, Plain{});
+            }
         } else if (a.small_structures) {
             // (weighted: float64 exps)
             if (f32) launch(F32{}, Small{}, Plain{});
