@@ -781,6 +781,7 @@ int mdx_hip_soap_plan_create(mdx_hip_ctx* ctx, const mdx_soap_params* params, md
                     plan->block_waves = bp.waves;
                     plan->block_kg = bp.kg;
                     plan->block_ncr = bp.ncr;
+                    plan->block_every_form = bp.every_form;
                     upload(plan->d_block_e1[f32], bp.lane_e1);
                     upload(plan->d_block_beta, bp.lane_beta);
                     upload(plan->d_block_ps[f32], bp.ps_offsets);

@@ -509,6 +509,7 @@ struct mdx_soap_plan {
     // coefficient registers, lane tables
     int block_waves = 0, block_kg = 0, block_ncr = 0;
     bool block_float32 = false; // float32 exps (block_float32_exps)
+    bool block_every_form = false; // BlockShape::every_form
     bool block_forced = false; // MDX_HIP_SOAP_KERNEL=block: also for inner averages of few large structures
     // exp constants and feature offsets with float64 [0] and float32 [1] exps,
     // those the plan may run

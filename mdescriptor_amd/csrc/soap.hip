@@ -471,14 +471,32 @@ Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph
     const bool outer_lds = p.average == 2 && whole && p.radial_basis == 0 && F * sizeof(double) <= static_cast<double>(kBlockOuterLdsBytes) &&
                            (!few || saving > kFastest);
     const bool outer_rows = static_cast<double>(pb.atoms) * F * 8.0 <= 4294967296.0;
-    // Three radial groups pad the power spectrum's Gram tiles (a register per
-    // species), which centres of few neighbours do not repay: 1,000 molecules
-    // of 9-29 atoms at n_max 10, l_max 7, 16x16 kernel and here: rows of five
-    // species 835 and 996 us (three: 502 and 425), outer averages of three
-    // 694 and 826, of five 1,325 and 1,439 (rows of condensed cells of five
-    // species 833 and 655)
-    const bool padded = p.block_kg == 3 && p.block_ncr >= (p.average == 2 ? 3 : 5) && p.average != 1 && p.use_mfma &&
-                        !p.block_forced && pb.most_images <= kBlockSmallAtoms;
+    // The power spectrum's Gram tiles are register pairs of 16 channels here,
+    // padded to whole radial groups, and pairs of 16 packed channels in the
+    // tile kernels; centres of few neighbours do not repay the padding.
+    // 1,000 molecules of 9-29 atoms, tile kernels and here (us):
+    //   three radial groups, n 10 l 7 (which also spill registers): rows of
+    //     five species 835 and 996 (three: 502 and 425; condensed cells of five
+    //     833 and 655), outer averages of three 694 and 826, of five 1,325 and
+    //     1,439
+    //   one group in two registers where one tile holds the channels (two
+    //     from l 8), default options: rows of five species n 2 l 6 146 and 192,
+    //     of eight n 1 l 9 0.64 of the rate (with 75-85 atoms 0.87, 115-125
+    //     0.96); of eight n 4 l 6 1.19
+    //   outer averages, at least twice the tile pairs, default options: five
+    //     species n 5 l 9 0.63 of the rate, l 6 493 and 580, l 2 1.27 of it (of
+    //     40-60 atoms 0.85; 75-85 1.5); shapes compiled in every form stay
+    //   mu1nu1 outer averages past l 8 of three registers: 850 and 1,047
+    const int64_t channels = static_cast<int64_t>(p.Sc) * p.n, packed = (channels + 15) / 16;
+    const bool twice = p.block_ncr * (p.block_ncr + 1) >= 2 * packed * (packed + 1);
+    const bool defaults = p.quad_waves > 0; // (else the tile kernel is the 16x16 one)
+    const bool padded =
+        p.use_mfma && !p.block_forced && p.average != 1 && pb.most_images <= kBlockSmallAtoms &&
+        (p.block_kg == 3 ? p.block_ncr >= (p.average == 2 ? 3 : 5)
+         : defaults && p.block_kg == 1 && p.block_ncr == 2 && channels <= (p.l_max >= 8 ? 18 : 16) ? true
+         : p.average == 2 && !p.block_every_form && defaults ? twice
+         : p.average == 2 && p.radial_basis == 0 && p.compression == 2 ? p.l_max > 8 && p.block_ncr >= 3
+                                                                       : false);
     const bool scratch_rows = p.weighted != 0 || p.radial_basis == 1;
     c.block = p.block_waves > 0 && (p.average != 2 || outer_rows || outer_lds) && !padded && g.row_bound < kQuadMaxRows &&
               !(saving == kLeast && scratch_rows && p.use_mfma && !p.block_forced);

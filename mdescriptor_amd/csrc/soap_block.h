@@ -108,6 +108,7 @@ struct BlockPlanHost {
     int kg = 0;      // radial groups of 4 channels
     int ncr = 0;     // coefficient registers per (l, column group)
     int waves = 0;   // wavefronts per workgroup
+    bool every_form = false; // BlockShape::every_form
     std::vector<double> lane_e1, lane_beta;
     std::vector<int32_t> ps_offsets; // packed feature offsets
 };

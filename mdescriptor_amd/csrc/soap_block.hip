@@ -193,6 +193,7 @@ bool block_plan_tables(int S, int n, int l_max, int table_dtype, int compression
     out.kg = kg;
     out.ncr = ncr;
     out.waves = e->waves;
+    out.every_form = e->every_form;
     return true;
 }
 

@@ -276,3 +276,28 @@ def test_float32_rows_of_float64_exps(hip_context, shape, average, name):
         if average == "inner" and name == "pow_w0" and sizes[0] > 64:
             continue  # a few large structures: float32 exps
         np.testing.assert_array_equal(rows["float32"], rows["float64"].astype(np.float32))
+
+
+@pytest.mark.parametrize("shape,average,compression", [
+    ((5, 2, 6), "off", "off"), ((8, 1, 9), "off", "off"), ((6, 3, 8), "off", "off"), ((5, 3, 2), "outer", "off"),
+    ((5, 5, 6), "outer", "off"), ((5, 8, 9), "outer", "mu1nu1"),
+])
+def test_molecules_of_padded_shapes(hip_context, oracle, shape, average, compression):
+    """Structures of few neighbours whose power spectrum this kernel would pad
+    take the tile kernels; larger ones of the same shape stay."""
+
+    count, n_max, l_max = shape
+    alphas, betas = basis_gto(4.0, n_max, l_max)
+    arguments = dict(species=SPECIES[:count], n_max=n_max, l_max=l_max, r_cut=4.0, sigma=1.0, alphas=alphas,
+                     betas=betas, average=average, options={"compression": compression} if compression != "off" else {})
+    plan = _hip.SoapPlan(hip_context, dtype="float64", **arguments)
+    try:
+        for sizes, block in (((21, 13, 1, 20), False), ((66, 70), True)):
+            batch = _structures(9, sizes, SPECIES[:count])
+            if not block:
+                batch.cells[:], batch.pbc[:] = 0.0, 0
+            values, timing = plan.compute(batch)
+            assert (timing["expansion_tiles"] <= -1000) == block
+            assert scaled_error(values, oracle.soap(batch, **arguments)) <= GATES["float64"]
+    finally:
+        plan.close()
