@@ -970,6 +970,13 @@ void settle(mdx_hip_ctx* ctx, mdx_device_batch* batch) {
     MDX_HIP(hipEventRecord(batch->done[j], s));
 }
 
+// Before work of ctx on the batch: on another context's streams than those of
+// the context it was uploaded on, which alone a kept batch waits for, it is
+// freed when it is destroyed.
+void note_streams(const mdx_hip_ctx* ctx, mdx_device_batch* batch) {
+    if (batch->spare != ctx->spare) batch->spare.reset();
+}
+
 // Settle the batch's pipelined frames and wait for them (their expansions
 // read its sets), so that a synchronous call may reuse set 0.
 void quiesce(mdx_hip_ctx* ctx, mdx_device_batch* batch) {
@@ -994,6 +1001,7 @@ int mdx_hip_batch_set_positions(mdx_hip_ctx* ctx, mdx_device_batch* batch, const
         if (values == 0) return;
         if (positions == nullptr) throw mdx::Error(MDX_INVALID_ARGUMENT, "null positions");
         DeviceScope scope(ctx->device);
+        note_streams(ctx, batch);
         quiesce(ctx, batch);
         if (is_device_memory(positions)) {
             // checked for finiteness by the next run's frame kernels
@@ -1023,7 +1031,7 @@ void mdx_hip_batch_destroy(mdx_device_batch* batch) {
 namespace {
 
 // Arguments of a device-batch run, checked as mdx_hip_soap_run documents.
-void check_device_run(const mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_device_batch* batch,
+void check_device_run(const mdx_hip_ctx* ctx, const mdx_soap_plan* plan, mdx_device_batch* batch,
                       const void* out_device, int64_t out_pitch_bytes) {
     if (plan == nullptr || batch == nullptr) throw mdx::Error(MDX_INVALID_ARGUMENT, "null plan or batch");
     if (plan->device != ctx->device || batch->device != ctx->device) {
@@ -1036,6 +1044,7 @@ void check_device_run(const mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const m
     const int64_t row_bytes = plan->features * plan->out_dtype;
     if (out_pitch_bytes < row_bytes) throw mdx::Error(MDX_INVALID_ARGUMENT, "output pitch is too small");
     if (rows > 0 && row_bytes > 0 && out_device == nullptr) throw mdx::Error(MDX_INVALID_ARGUMENT, "null output");
+    note_streams(ctx, batch);
 }
 
 } // namespace
@@ -1162,6 +1171,7 @@ int mdx_hip_batch_wait(mdx_hip_ctx* ctx, mdx_device_batch* batch) {
         if (batch == nullptr) throw mdx::Error(MDX_INVALID_ARGUMENT, "null batch");
         if (batch->device != ctx->device) throw mdx::Error(MDX_INVALID_ARGUMENT, "batch belongs to another device");
         DeviceScope scope(ctx->device);
+        note_streams(ctx, batch); // (a frame to settle may run again here)
         quiesce(ctx, batch);
     });
 }

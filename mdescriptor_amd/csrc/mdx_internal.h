@@ -436,7 +436,8 @@ namespace mdx {
 // and destroys it (SOAP.compute_into) then allocates nothing after the first
 // (35 device and two pinned allocations and their frees, 0.3 ms a call, up to
 // 1.6 ms for 20,000 structures).  Idle: its work has finished, and it belongs
-// to no caller.  Freed with the context, or when a device allocation fails.
+// to no caller.  A batch that another context's streams have worked on is not
+// kept.  Freed with the context, or when a device allocation fails.
 struct SpareBatch {
     std::mutex mutex;
     bool open = true; // false once the context is going

@@ -522,3 +522,55 @@ def test_destroyed_batches_leave_nothing_to_the_next(hip_context, oracle):
     for batch, plan in kept:
         batch.close()
         plan.close()
+
+
+def _free_device_bytes() -> int:
+    runtime = _hip.DeviceMemory.runtime()
+    runtime.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]
+    runtime.hipMemGetInfo.restype = ctypes.c_int
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert runtime.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return int(free.value)
+
+
+def _large(atoms=40000):
+    rng = np.random.default_rng(6)
+    side = int(np.ceil(atoms ** (1.0 / 3.0)))
+    sites = np.stack(np.unravel_index(rng.permutation(side ** 3)[:atoms], (side,) * 3), axis=1)
+    return SimpleNamespace(numbers=np.resize([1, 8], atoms).astype(np.int32),
+                           positions=sites * 2.15 + rng.uniform(-0.2, 0.2, (atoms, 3)),
+                           cells=np.eye(3)[None] * side * 2.15, pbc=np.ones((1, 3), np.int32),
+                           offsets=np.array([0, atoms], np.int64))
+
+
+def test_batch_run_on_another_context_is_freed():
+    """A batch uploaded on one context and run on another (whose streams the
+    first does not wait for) is not kept for the first's next upload."""
+
+    params = {"species": [1, 8], "n_max": 2, "l_max": 2, "r_cut": 4.0}
+    owner, other = _hip.Context(0), _hip.Context(0)
+    plan, _ = _plan(owner, params, "off", "float64")
+    foreign, _ = _plan(other, params, "off", "float64")
+    work = _large()
+    try:
+        before = _free_device_bytes()
+        batch = _Resident(plan, work)
+        rows, _ = batch.run()
+        ctx = other
+        for _ in range(2):
+            ctx.check(ctx.lib.mdx_hip_soap_run_frame(ctx.handle, foreign.handle, batch.batch.handle,
+                                                     np.ascontiguousarray(work.positions).ctypes.data_as(ctypes.c_void_p),
+                                                     ctypes.c_void_p(batch.out.address), batch.pitch, None))
+        batch.batch.close()  # frames still queued on the other context
+        assert before - _free_device_bytes() < (64 << 20) + rows.nbytes
+        after = _Resident(plan, _moved(work, work.positions + 3.0))
+        after.run()
+        np.testing.assert_array_equal(batch.out.to_host(np.empty_like(rows)), rows)
+        after.batch.close()
+        after.out.free()
+        batch.out.free()
+    finally:
+        plan.close()
+        foreign.close()
+        owner.close()
+        other.close()
