@@ -175,8 +175,10 @@ int mdx_hip_soap_compute(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_
  * (the H2D part of Backend::compute, cpp/cuda/src/backend.cu:353-356) */
 int mdx_hip_batch_upload(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_batch_view* batch,
                          mdx_device_batch** out);
-/* The context keeps one destroyed batch's buffers (at most 1 GiB) for the next
- * upload; they are freed with the context or when an allocation fails. */
+/* The context keeps one destroyed batch's buffers (at most 1 GiB, and past 16
+ * MiB at most 1/64 of the device's free memory) for the next upload of about
+ * its size; they are freed with the context or when one of the library's
+ * allocations fails. */
 void mdx_hip_batch_destroy(mdx_device_batch* batch);
 
 /* New positions for a device-resident batch (a new frame of the same system:

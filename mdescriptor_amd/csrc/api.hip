@@ -409,7 +409,15 @@ void download_result(mdx_hip_ctx* ctx, const void* src, int64_t rows, int64_t ro
 
 namespace mdx {
 
-mdx_device_batch* SpareBatch::take() {
+mdx_device_batch* SpareBatch::take(int64_t atoms) {
+    std::lock_guard<std::mutex> lock(mutex);
+    if (batch != nullptr && batch->pb.atoms / kSpareAtoms > atoms && batch_bytes(*batch) > kSpareSmallBytes) return nullptr;
+    mdx_device_batch* b = batch;
+    batch = nullptr;
+    return b;
+}
+
+mdx_device_batch* SpareBatch::release() {
     std::lock_guard<std::mutex> lock(mutex);
     mdx_device_batch* b = batch;
     batch = nullptr;
@@ -417,7 +425,12 @@ mdx_device_batch* SpareBatch::take() {
 }
 
 bool SpareBatch::keep(mdx_device_batch* returned) {
-    if (batch_bytes(*returned) > kSpareBytes) return false;
+    const size_t held = batch_bytes(*returned);
+    if (held > kSpareBytes) return false;
+    if (held > kSpareSmallBytes) {
+        size_t free = 0, total = 0;
+        if (hipMemGetInfo(&free, &total) != hipSuccess || free / kSpareFreeShare < held) return false;
+    }
     mdx_device_batch* old = nullptr;
     {
         std::lock_guard<std::mutex> lock(mutex); // (the context waits for it before its streams go)
@@ -430,7 +443,7 @@ bool SpareBatch::keep(mdx_device_batch* returned) {
 }
 
 bool SpareBatch::drop() {
-    mdx_device_batch* b = take();
+    mdx_device_batch* b = release();
     delete b;
     return b != nullptr;
 }
@@ -915,7 +928,7 @@ int mdx_hip_batch_upload(mdx_hip_ctx* ctx, const mdx_soap_plan* plan, const mdx_
         if (plan == nullptr || batch == nullptr) throw mdx::Error(MDX_INVALID_ARGUMENT, "null plan or batch");
         if (plan->device != ctx->device) throw mdx::Error(MDX_INVALID_ARGUMENT, "plan belongs to another device");
         DeviceScope scope(ctx->device);
-        mdx_device_batch* db = ctx->spare->take();
+        mdx_device_batch* db = ctx->spare->take(batch->atoms);
         if (db == nullptr) db = new mdx_device_batch();
         try {
             db->device = ctx->device;

@@ -436,19 +436,27 @@ namespace mdx {
 // and destroys it (SOAP.compute_into) then allocates nothing after the first
 // (35 device and two pinned allocations and their frees, 0.3 ms a call, up to
 // 1.6 ms for 20,000 structures).  Idle: its work has finished, and it belongs
-// to no caller.  A batch that another context's streams have worked on is not
-// kept.  Freed with the context, or when a device allocation fails.
+// to no caller.  Only an upload of about its size takes it (a small batch that
+// stays resident would hold a large one's buffers, out of reach of the bound
+// and of a failed allocation), and a large one is kept only while the device
+// has plenty of memory free, since other allocators cannot ask for it back.
+// A batch that another context's streams have worked on is not kept.  Freed
+// with the context, or when a device allocation fails.
 struct SpareBatch {
     std::mutex mutex;
     bool open = true; // false once the context is going
     hipStream_t streams[3] = {}; // the context's
     mdx_device_batch* batch = nullptr;
-    mdx_device_batch* take();              // the spare (the caller's now), or null
+    mdx_device_batch* take(int64_t atoms); // the spare for an upload of that many atoms (the caller's now), or null
+    mdx_device_batch* release();           // the spare whatever its size, or null
     bool keep(mdx_device_batch* returned); // false: not kept (the caller deletes it)
     bool drop();                           // frees the spare; true if there was one
     ~SpareBatch();
 };
 constexpr size_t kSpareBytes = size_t(1) << 30;
+constexpr size_t kSpareSmallBytes = size_t(16) << 20; // any upload may take
+constexpr int64_t kSpareAtoms = 4;   // ... else one of at least a quarter of its atoms
+constexpr size_t kSpareFreeShare = 64; // kept while at least this many times its bytes are free
 // Every context's spare freed; true if memory came back (device allocations
 // retry then).
 bool drop_spare_batches();

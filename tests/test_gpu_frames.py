@@ -543,6 +543,38 @@ def _large(atoms=40000):
                            offsets=np.array([0, atoms], np.int64))
 
 
+def test_kept_buffers_go_to_a_batch_of_their_size(oracle):
+    """A small batch that stays resident leaves a large destroyed batch's
+    buffers to the next large one."""
+
+    params = {"species": [1, 8], "n_max": 2, "l_max": 2, "r_cut": 4.0}
+    context = _hip.Context(0)
+    plan, basis = _plan(context, params, "off", "float64")
+    work = _large()
+    small = _moved(work, work.positions)
+    small.numbers, small.positions = work.numbers[:50], work.positions[:50]
+    small.cells, small.pbc, small.offsets = np.zeros((1, 3, 3)), np.zeros((1, 3), np.int32), np.array([0, 50])
+    try:
+        before = _free_device_bytes()
+        first = _Resident(plan, work)
+        rows, _ = first.run()
+        held = before - _free_device_bytes() - first.batch.rows * first.pitch
+        assert held > 100 << 20
+        first.close()
+        resident = _Resident(plan, small)
+        second = _Resident(plan, work)
+        again, _ = second.run()
+        np.testing.assert_array_equal(again, rows)
+        assert before - _free_device_bytes() - second.batch.rows * second.pitch < 1.5 * held
+        few, _ = resident.run()
+        assert scaled_error(few, _oracle_soap(oracle, small, params, basis, "off")) <= F64_GATE
+        resident.close()
+        second.close()
+    finally:
+        plan.close()
+        context.close()
+
+
 def test_batch_run_on_another_context_is_freed():
     """A batch uploaded on one context and run on another (whose streams the
     first does not wait for) is not kept for the first's next upload."""
