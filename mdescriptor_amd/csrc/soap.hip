@@ -21,26 +21,13 @@
 #include "mdx_internal.h"
 #include "soap_mfma.h"
 #include "soap_block.h"
+#include "soap_choice.h"
 
 #include <algorithm>
 #include <cmath>
-#include <limits>
 
 namespace mdx {
 
-constexpr int kItemCentres = 32;
-// polynomial basis: bytes of radial functions a slice of centres holds, at
-// most (what the last-level cache keeps between the two kernels of a slice)
-constexpr int64_t kPolySliceBytes = int64_t(256) << 20;
-// ... and the fewest centres of a slice: with less room the 16x16 kernel forms
-// the functions itself (as fast as slices of 128 centres on the register-
-// coefficient kernel: 3,000 atoms, n 6 l 5, 1,255 us, in slices of 128, 256
-// and 1,024 centres 1,221, 840 and 507; n 3 l 2, 639 and 756, 522, 325).  By
-// row as many as give the device 2,048 wavefronts, one per centre and tile
-// (n 4 l 1, a tile: 662 us, in slices of 512, 1,024 and 3,000 centres 1,071,
-// 691 and 524; n 3 l 10, eight tiles: 5,751 us, of 256 centres 1,331)
-constexpr int64_t kPolyLeastCentres = 256, kPolyLeastWaves = 2048;
-constexpr size_t kPolySlack = 4096; // alignment of the scratch's parts
 constexpr int kFoldItems = 16;  // rows per split, at least
 constexpr int kFoldSplits = 32; // splits per structure, at most
 
@@ -60,20 +47,6 @@ int64_t partial_budget(const PreparedBatch& pb, const DeviceGraph& g, bool weigh
     constexpr double kArray = static_cast<double>(MDX_NOALLOC_SCRATCH_BYTES);
     if (graph > 1.25 * kArray) return int64_t(1) << 30;
     return std::max<int64_t>(0, static_cast<int64_t>(0.85 * kArray - graph));
-}
-
-// Centres per run of an averaged structure: kItemCentres where the batch then
-// still has a few runs for every compute unit, shorter for smaller batches
-// (8,192 atoms at 32 are 256 runs, one workgroup a compute unit) as far as
-// their partial rows (width doubles each, and the folded ones) fit the budget.
-int64_t run_centres(const PreparedBatch& pb, size_t width, int64_t budget) {
-    const int64_t fill = 8 * static_cast<int64_t>(device_compute_units());
-    int64_t length = std::max<int64_t>(1, std::min<int64_t>(kItemCentres, pb.atoms / fill));
-    auto bytes = [&](int64_t len) {
-        return static_cast<double>(pb.atoms / len + 33 * pb.structures) * static_cast<double>(width) * sizeof(double);
-    };
-    while (length < kItemCentres && bytes(length) > static_cast<double>(budget)) length *= 2;
-    return std::min<int64_t>(length, kItemCentres);
 }
 
 // Pair rows of the graph's layout.
@@ -424,134 +397,6 @@ void dispatch_hpt(int hpt, hipStream_t stream, dim3 grid, size_t lds, const mdx_
     }
 }
 
-// The kernel and the decomposition of a run.
-struct Choice {
-    bool block = false;           // the register-coefficient kernel
-    bool block_inner = false;     // ... a workgroup per structure
-    bool block_runs = false;      // ... runs of a structure's centres into partial coefficient rows
-    bool block_outer = false;     // ... a float64 partial row per centre
-    bool block_outer_lds = false; // ... a workgroup per structure, power spectra summed in LDS
-    bool f32_exps = false;        // ... with float32 exps
-    bool quad = false;            // the 4x4-block kernel
-    bool poly_inside = false;     // polynomial basis: radial functions in the 16x16 kernel, without scratch
-    int64_t largest_structure = 0;
-    int64_t run = kItemCentres;   // centres per run
-    size_t partial_width = 0;     // doubles of a partial row
-    bool partials() const { return !block_inner && !block_outer_lds; } // (of an average)
-};
-
-// Scratch a run may save: kFastest, no more of it than runs of kItemCentres
-// take, none for the register-coefficient kernel's partial rows, none beside
-// the other kernels' partial rows (no row weights, no radial functions).
-constexpr int kFastest = 0, kLongRuns = 1, kShortRows = 2, kLeast = 3;
-Choice choose(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g, int64_t budget, int saving) {
-    Choice c;
-    const double F = static_cast<double>(p.features);
-    for (size_t st = 0; st + 1 < pb.offsets.size(); ++st) {
-        c.largest_structure = std::max(c.largest_structure, pb.offsets[st + 1] - pb.offsets[st]);
-    }
-    const int64_t units = device_compute_units();
-    // The register-coefficient kernel where the plan chose it and every
-    // centre's rows fit their slot codes.  It forms a structure's average in
-    // one workgroup when the structures are small (a wavefront of atoms) or
-    // many enough to fill the device (four per compute unit); the inner
-    // averages of a few large structures (16 cells of 4,096 atoms: 16
-    // workgroups, 50 ms) sum runs of centres into partial coefficient rows
-    // instead, reduced per structure (1.1 ms).
-    const bool whole = c.largest_structure <= kBlockSmallAtoms || p.block_forced || pb.structures >= 4 * units;
-    // Outer averages with a workgroup per structure add each centre's power
-    // spectrum into the structure's float64 row in LDS and write the mean
-    // once, with no partial rows in HBM.  Large structures, and rows past the
-    // LDS, take every centre's row as a float64 partial row (at most 4 GiB of
-    // them), folded per structure, then the mean (k_finalize_outer); so do
-    // fewer structures than two per compute unit, which spread over the
-    // device better, where the scratch allows.
-    const double centre_rows = static_cast<double>(pb.atoms + 5 * pb.structures) * F * 8.0;
-    const bool few = pb.structures < 2 * units && centre_rows <= static_cast<double>(budget);
-    const bool outer_lds = p.average == 2 && whole && p.radial_basis == 0 && F * sizeof(double) <= static_cast<double>(kBlockOuterLdsBytes) &&
-                           (!few || saving > kFastest);
-    const bool outer_rows = static_cast<double>(pb.atoms) * F * 8.0 <= 4294967296.0;
-    // The power spectrum's Gram tiles are register pairs of 16 channels here,
-    // padded to whole radial groups, and pairs of 16 packed channels in the
-    // tile kernels; centres of few neighbours do not repay the padding.
-    // 1,000 molecules of 9-29 atoms, tile kernels and here (us):
-    //   three radial groups, n 10 l 7 (which also spill registers): rows of
-    //     five species 835 and 996 (three: 502 and 425; condensed cells of five
-    //     833 and 655), outer averages of three 694 and 826, of five 1,325 and
-    //     1,439
-    //   one group in two registers where one tile holds the channels (two
-    //     from l 8), default options: rows of five species n 2 l 6 146 and 192,
-    //     of eight n 1 l 9 0.64 of the rate (with 75-85 atoms 0.87, 115-125
-    //     0.96); of eight n 4 l 6 1.19
-    //   outer averages, at least twice the tile pairs, default options: five
-    //     species n 5 l 9 0.63 of the rate, l 6 493 and 580, l 2 1.27 of it (of
-    //     40-60 atoms 0.85; 75-85 1.5); shapes compiled in every form stay
-    //   mu1nu1 outer averages past l 8 of three registers: 850 and 1,047
-    const int64_t channels = static_cast<int64_t>(p.Sc) * p.n, packed = (channels + 15) / 16;
-    const bool twice = p.block_ncr * (p.block_ncr + 1) >= 2 * packed * (packed + 1);
-    const bool defaults = p.quad_waves > 0; // (else the tile kernel is the 16x16 one)
-    const bool padded =
-        p.use_mfma && !p.block_forced && p.average != 1 && pb.most_images <= kBlockSmallAtoms &&
-        (p.block_kg == 3 ? p.block_ncr >= (p.average == 2 ? 3 : 5)
-         : defaults && p.block_kg == 1 && p.block_ncr == 2 && channels <= (p.l_max >= 8 ? 18 : 16) ? true
-         : p.average == 2 && !p.block_every_form && defaults ? twice
-         : p.average == 2 && p.radial_basis == 0 && p.compression == 2 ? p.l_max > 8 && p.block_ncr >= 3
-                                                                       : false);
-    const bool scratch_rows = p.weighted != 0 || p.radial_basis == 1;
-    c.block = p.block_waves > 0 && (p.average != 2 || outer_rows || outer_lds) && !padded && g.row_bound < kQuadMaxRows &&
-              !(saving == kLeast && scratch_rows && p.use_mfma && !p.block_forced);
-    // By row the radial functions come a species at a time, padded to tiles of
-    // 16 rows; the 16x16 kernel forms those of 32 rows at once.  It is the
-    // faster of the two for up to eight degrees and channels (past them it
-    // meets a barrier every four grid points: from memory 2.6-6 times as
-    // fast) with more than six species, or three to six that do not fill two
-    // tiles each.  l 1, n 4, from memory and inside: 4,000 condensed atoms of
-    // two, four, six, ten species 604 and 830 us, 674 and 825, 822 and 870, 953
-    // and 922; 2,000 molecules of 9-29 atoms of two, three, six species 753 and
-    // 958, 1,313 and 1,067, 1,709 and 1,384; l 2 n 6, 4,000 atoms of nine 1,276
-    // and 1,024.
-    const bool short_tiles = p.S > 6 || (p.S > 2 && std::min(pb.most_images, g.row_bound) < 32 * p.S);
-    c.poly_inside = p.radial_basis == 1 && !c.block && (saving == kLeast || (p.L <= 8 && p.n <= 8 && short_tiles));
-    const size_t block_width = c.block ? static_cast<size_t>(block_partial_width(p.l_max, p.block_ncr)) : 0;
-    // A few small periodic structures hold thousands of pairs each (a
-    // workgroup takes about a microsecond per 32 of them): runs too.
-    const bool spread = saving == kFastest && !p.block_forced && pb.structures < units &&
-                        c.largest_structure * std::min(pb.most_images, g.row_bound) > kBlockSpreadPairs &&
-                        static_cast<double>(pb.atoms + 5 * pb.structures) * static_cast<double>(block_width) * 8.0 <=
-                            static_cast<double>(budget);
-    // Centres of the polynomial basis that a slice of radial functions holds.
-    // A structure formed in one workgroup needs all of its centres at once: one
-    // past that (12,000 atoms among 1,024 molecules: 1.2 GB at l 2) sums runs,
-    // and no run is longer.
-    const PolyLayout poly = poly_layout(g.row_bound, p.S, p.L, p.n, c.block);
-    const int64_t slice_centres =
-        p.radial_basis != 1 || c.poly_inside
-            ? std::numeric_limits<int64_t>::max()
-            : std::max<int64_t>(1, kPolySliceBytes / (poly.centre * static_cast<int64_t>(sizeof(double))));
-    // (weighted inner averages: those of few large structures only, whose
-    // former kernel had them)
-    c.f32_exps = c.block && p.block_float32 && !(p.average == 1 && p.weighted != 0 && whole);
-    c.block_inner = c.block && p.average == 1 && whole && !spread && c.largest_structure <= slice_centres;
-    c.block_outer_lds = c.block && outer_lds;
-    c.block_runs = c.block && p.average == 1 && !c.block_inner;
-    c.block_outer = c.block && p.average == 2 && !outer_lds;
-    if (saving >= kShortRows && (c.block_runs || c.block_outer) && !p.block_forced) {
-        c.block = c.block_runs = c.block_outer = false;
-    }
-    // else the 4x4-block kernel where the plan chose it (its coefficient rows
-    // are its own), the 16x16 kernel, the generic one
-    c.quad = !c.block && p.use_mfma && p.quad_waves > 0 && g.row_bound < kQuadMaxRows;
-    const int rows = c.quad ? quad_coefficient_rows(p.Sc, p.n) : mfma_coefficient_rows(p.Sc, p.n, p.compression);
-    c.partial_width = c.block_runs     ? block_width
-                      : p.average != 1 ? static_cast<size_t>(p.features)
-                      : p.use_mfma     ? static_cast<size_t>(rows) * static_cast<size_t>(p.hpad)
-                                       : static_cast<size_t>(p.coeff_size);
-    if (p.average != 0 && c.partials() && !c.block_outer) {
-        c.run = std::min<int64_t>(slice_centres, saving == kFastest ? run_centres(pb, c.partial_width, budget) : kItemCentres);
-    }
-    return c;
-}
-
 // Bytes of the folded rows' splits: see k_fold_partials.
 struct Fold {
     int splits = 0;
@@ -566,19 +411,42 @@ Fold fold_of(int64_t most_items) {
     return f;
 }
 
-// The polynomial basis' radial functions of a run.
-PolyLayout poly_layout_of(const mdx_soap_plan& p, const DeviceGraph& g, const Choice& c) {
-    if (p.radial_basis != 1 || c.poly_inside) return {};
-    return poly_layout(g.row_bound, p.S, p.L, p.n, c.block);
-}
-
-// The least scratch for them: a slice's centres, at least an item's.
-size_t poly_least_bytes(const mdx_soap_plan& p, const PreparedBatch& pb, const PolyLayout& layout, const Choice& c) {
-    if (layout.centre == 0) return 0;
-    const int64_t item = c.block_inner ? c.largest_structure : p.average != 0 && !c.block_outer ? c.run : 1;
-    const int64_t slice = c.block ? kPolyLeastCentres : std::max(kPolyLeastCentres, kPolyLeastWaves / p.tiles);
-    const int64_t centres = std::min(pb.atoms, std::max(item, slice));
-    return static_cast<size_t>(centres * layout.centre) * sizeof(double) + kPolySlack;
+static_assert(kSlotCodeRows == kQuadMaxRows, "one limit for both 4x4 kernels");
+ChoiceInput choice_input(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g) {
+    ChoiceInput in;
+    in.average = p.average;
+    in.radial_basis = p.radial_basis;
+    in.compression = p.compression;
+    in.weighted = p.weighted;
+    in.S = p.S;
+    in.Sc = p.Sc;
+    in.n = p.n;
+    in.L = p.L;
+    in.l_max = p.l_max;
+    in.features = p.features;
+    in.use_mfma = p.use_mfma;
+    in.tiles = p.tiles;
+    in.quad_waves = p.quad_waves;
+    in.block_waves = p.block_waves;
+    in.block_kg = p.block_kg;
+    in.block_ncr = p.block_ncr;
+    in.block_forced = p.block_forced;
+    in.block_float32 = p.block_float32;
+    in.block_every_form = p.block_every_form;
+    if (p.block_waves > 0) in.block_width = static_cast<size_t>(block_partial_width(p.l_max, p.block_ncr));
+    in.quad_width = static_cast<size_t>(quad_coefficient_rows(p.Sc, p.n)) * static_cast<size_t>(p.hpad);
+    in.tile_width = p.use_mfma ? static_cast<size_t>(mfma_coefficient_rows(p.Sc, p.n, p.compression)) * static_cast<size_t>(p.hpad)
+                               : static_cast<size_t>(p.coeff_size);
+    in.structures = pb.structures;
+    in.atoms = pb.atoms;
+    for (size_t st = 0; st + 1 < pb.offsets.size(); ++st) {
+        in.largest_structure = std::max(in.largest_structure, pb.offsets[st + 1] - pb.offsets[st]);
+    }
+    in.most_images = pb.most_images;
+    in.row_bound = g.row_bound;
+    in.units = device_compute_units();
+    in.budget = partial_budget(pb, g, p.weighted != 0);
+    return in;
 }
 
 // Scratch of a run beside the radial functions: its partial rows, folded
@@ -631,23 +499,22 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
         return;
     }
 
-    const int64_t budget = partial_budget(pb, g, p.weighted != 0);
-    Choice choice = choose(p, pb, g, budget, kFastest);
+    const ChoiceInput in = choice_input(p, pb, g);
+    Choice choice = choose(in, kFastest);
     if (partials.arena != nullptr) {
         // the static array of a no-allocation run: what does not fit there
         // takes long runs, then the tile kernels' short partial rows, then
         // those kernels without row weights or radial functions in memory
         const size_t room = partials.arena->left() + partials.bytes;
         auto fits = [&](const Choice& c) {
-            return scratch_bytes(p, pb, g, c) + poly_least_bytes(p, pb, poly_layout_of(p, g, c), c) <= room;
+            return scratch_bytes(p, pb, g, c) + poly_least_bytes(in, c) <= room;
         };
         for (int saving = kLongRuns; saving <= kLeast && !fits(choice); ++saving) {
-            choice = choose(p, pb, g, budget, saving);
+            choice = choose(in, saving);
         }
     }
     const bool block = choice.block, block_inner = choice.block_inner, block_runs = choice.block_runs;
     const bool block_outer = choice.block_outer, block_outer_lds = choice.block_outer_lds;
-    const int64_t largest_structure = choice.largest_structure;
     const size_t partial_width = choice.partial_width;
 
     // work items
@@ -696,7 +563,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
     };
     int64_t poly_centres = 0;
     size_t poly_bytes = 0;
-    const PolyLayout layout = poly_layout_of(p, g, choice);
+    const PolyLayout layout = poly_layout_of(in, choice);
     if (layout.centre > 0) {
         const int64_t centre_bytes = layout.centre * static_cast<int64_t>(sizeof(double));
         int64_t room = kPolySliceBytes;
@@ -899,8 +766,7 @@ void run_soap(hipStream_t stream, const mdx_soap_plan& p, PreparedBatch& pb, con
                                                                   : nullptr;
                 ba.outer_lds = block_outer_lds ? 1 : 0;
                 ba.partial_out = block_runs ? d_partial : nullptr;
-                ba.small_structures =
-                    block_inner && largest_structure <= kBlockSmallAtoms && p.radial_basis == 0 ? 1 : 0;
+                ba.small_structures = choice.block_small ? 1 : 0;
                 ba.summed = p.compression == 2 ? 1 : 0;
                 ba.mu2 = p.compression == 1 ? 1 : 0;
                 // without weights every species weight is 1

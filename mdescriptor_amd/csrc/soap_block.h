@@ -6,6 +6,7 @@
 #pragma once
 
 #include "mdx_internal.h"
+#include "soap_choice.h"
 
 namespace mdx {
 
@@ -34,12 +35,6 @@ constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuter
 // own type (shapes compiled in every form).
 constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2, kBlockHalf = 3, kBlockWeightedRows = 4;
 constexpr int kBlockPolyGroups = 2;
-// largest row (features x 8 bytes) the outer mode accumulates in LDS
-constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;
-constexpr int kBlockSmallAtoms = 64;
-// pairs of a structure past which a batch of fewer structures than compute
-// units sums runs of its centres instead of whole structures
-constexpr int64_t kBlockSpreadPairs = 4096;
 
 // Launch arguments (one struct, passed by value).
 struct BlockArgs {

@@ -2,10 +2,11 @@
 
 Every number of radial groups (n_max 1-4, 5-8, 9-12) with every number of
 coefficient registers, exactly filled and rounded up to the next compiled
-one, at the smallest and largest l_max and in between; each average on
-structures of at most a wavefront of atoms and on larger ones; neighbour
-weights and every compression.  Gates as in test_gpu_parity.py: float64
-|delta| <= 1e-10 (|ref| + max|row|), float32 the same form at 2e-5.
+one, at the smallest and largest l_max and in between, with each average;
+every mode of an average (which the run's own rule, evaluated on the host,
+says a batch takes), neighbour weights and every compression.  Gates as in
+test_gpu_parity.py: float64 |delta| <= 1e-10 (|ref| + max|row|), float32 the
+same form at 2e-5.
 """
 
 from __future__ import annotations
@@ -16,6 +17,7 @@ from types import SimpleNamespace
 import numpy as np
 import pytest
 
+import run_choice
 from conftest import scaled_error
 from mdescriptor_amd import _hip
 from mdescriptor_amd.descriptors.basis import basis_gto, basis_polynomial
@@ -77,8 +79,8 @@ def _check(ctx, oracle, batch, shape, average, dtype, options=None):
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("average", ["off", "inner", "outer"])
 def test_shape(hip_context, oracle, shape, average):
-    # 21 atoms a structure and a lone atom; then structures past a wavefront,
-    # which an average takes as runs or partial rows
+    # 21 atoms a structure (periodic ones among them) and a lone atom; then
+    # structures past a wavefront: averages as runs or centre rows, all of them
     for sizes, dtype in (((21, 13, 1, 20), "float64"), ((70, 66), "float32")):
         _check(hip_context, oracle, _structures(sum(shape), sizes, SPECIES[:shape[0]]), shape, average, dtype)
 
@@ -98,6 +100,50 @@ def test_shape_options(hip_context, oracle, shape, average, name):
         _check(hip_context, oracle, _structures(sum(shape), sizes, SPECIES[:shape[0]]), shape, average, dtype, options)
 
 
+def _clusters(seed, sizes, species):
+    """Isolated clusters only: few neighbours a structure."""
+
+    batch = _structures(seed, sizes, species)
+    batch.cells[:], batch.pbc[:] = 0.0, 0
+    return batch
+
+
+@pytest.fixture(scope="module")
+def run_rule(tmp_path_factory):
+    return run_choice.compiled(tmp_path_factory.mktemp("run_choice"))
+
+
+# structures of each mode of an average; forced: MDX_HIP_SOAP_KERNEL=block,
+# under which structures past a wavefront are formed whole however few
+MODES = {
+    "species-major structures": ("inner", (21, 13, 1, 20), False),
+    "whole structures": ("inner", (70, 66), True),
+    "runs": ("inner", (70, 66), False),
+    "centre rows": ("outer", (21, 13, 1, 20), False),
+    "rows in LDS": ("outer", (5, 1, 7, 4, 6) * 104, False),
+}
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 2), (8, 4, 5), (3, 8, 7), (4, 7, 3), (2, 9, 5), (5, 6, 4), (4, 8, 6)])
+@pytest.mark.parametrize("mode", sorted(MODES))
+@pytest.mark.parametrize("name", ["default", "pow_w0", "mu2", "mu1nu1", "crossover", "pow_w0_mu1nu1"])
+def test_modes_of_an_average(hip_context, oracle, run_rule, monkeypatch, shape, mode, name):
+    average, sizes, forced = MODES[mode]
+    options = dict(POW_W0) if "pow_w0" in name else {}
+    if name.split("_")[-1] in ("mu2", "mu1nu1", "crossover"):
+        options["compression"] = name.split("_")[-1]
+    if forced:
+        monkeypatch.setenv("MDX_HIP_SOAP_KERNEL", "block")
+    count, n_max, l_max = shape
+    batch = _clusters(sum(shape), sizes, SPECIES[:count])
+    for dtype in ("float64", "float32"):
+        plan = run_choice.plan_values(count, n_max, l_max, average, dtype, options)
+        plan["block_forced"] = forced
+        r_cut = 6.0 if n_max > 8 else 4.0
+        assert run_choice.mode(run_rule, plan, run_choice.batch_values(batch, r_cut)) == mode
+        _check(hip_context, oracle, batch, shape, average, dtype, options)
+
+
 def test_outer_average_past_the_lds_row(hip_context, oracle):
     """Small structures whose row is too wide for the LDS accumulation (more
     than 48 KB): a float64 partial row per centre."""
@@ -108,11 +154,11 @@ def test_outer_average_past_the_lds_row(hip_context, oracle):
 @pytest.mark.parametrize("shape", [
     (1, 1, 2), (4, 4, 3), (5, 3, 7), (2, 5, 2), (4, 5, 5), (5, 5, 6), (3, 4, 9),  # radial functions in step groups
     (2, 4, 1), (3, 3, 10), (8, 2, 11),                                 # by row, for the 16x16 kernel
-    (3, 4, 1), (6, 8, 0), (7, 5, 3), (8, 6, 4),                        # in that kernel (few rows a species, or many species)
+    (3, 4, 1), (6, 8, 0), (7, 5, 3), (8, 6, 4),                        # in that kernel (clusters, or many species)
 ])
 @pytest.mark.parametrize("average", ["off", "inner", "outer"])
 @pytest.mark.parametrize("name", ["default", "pow_w0", "mu1nu1"])
-def test_polynomial_basis(hip_context, oracle, shape, average, name):
+def test_polynomial_basis(hip_context, oracle, run_rule, shape, average, name):
     """Radial functions computed before the expansion, for the kernel that
     reads them in step groups and for the one that reads them by row; a lone
     atom (only the pair at distance zero), weights and a compression."""
@@ -121,8 +167,9 @@ def test_polynomial_basis(hip_context, oracle, shape, average, name):
     species = SPECIES[:count]
     options = {"default": {}, "pow_w0": dict(POW_W0), "mu1nu1": {"compression": "mu1nu1"}}[name]
     options["polynomial"] = basis_polynomial(4.0, n_max)
-    for sizes, dtype in (((21, 13, 1, 20), "float64"), ((70, 66), "float32")):
-        batch = _structures(sum(shape), sizes, species)
+    for build, sizes, dtype in ((_structures, (21, 13, 1, 20), "float64"), (_structures, (70, 66), "float32"),
+                                (_clusters, (21, 13, 1, 20), "float64")):
+        batch = build(sum(shape), sizes, species)
         arguments = dict(species=species, n_max=n_max, l_max=l_max, r_cut=4.0, sigma=1.0, alphas=None, betas=None,
                          average=average, options=options)
         plan = _hip.SoapPlan(hip_context, dtype=dtype, **arguments)
@@ -131,6 +178,11 @@ def test_polynomial_basis(hip_context, oracle, shape, average, name):
         finally:
             plan.close()
         assert (timing["expansion_tiles"] <= -1000) == (2 <= l_max <= 9 and (n_max <= 4 or count <= 6))
+        # radial functions in step groups, by row, or in the 16x16 kernel
+        values_in = {**run_choice.plan_values(*shape, average, dtype, options), **run_choice.batch_values(batch, 4.0)}
+        choice = run_choice.evaluate(run_rule, values_in)
+        assert choice["poly_inside"] == (shape in ((3, 4, 1), (6, 8, 0), (7, 5, 3), (8, 6, 4)) and
+                                         (count > 6 or values_in["row_bound"] < 32 * count))
         expected = oracle.soap(batch, **arguments)
         assert values.shape == expected.shape
         assert np.all(np.isfinite(values))
