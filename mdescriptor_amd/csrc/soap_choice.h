@@ -139,8 +139,14 @@ inline Choice choose(const ChoiceInput& in, int saving) {
          : in.average == 2 && !in.block_every_form && defaults ? twice
          : in.average == 2 && in.radial_basis == 0 && in.compression == 2 ? in.l_max > 8 && in.block_ncr >= 3
                                                                        : false);
+    // Rows in LDS of too few structures to fill the device, where their centre
+    // rows do not fit: the tile kernels' runs of centres fill it (150
+    // structures of 40-60 atoms, n 12 l 7 of two species, 475 us and 705; 30,
+    // n 8 l 9 of four, 458 and 549; 300, n 12 l 7, 761 and 825)
+    const bool underfilled = outer_lds && saving == kFastest && in.use_mfma && !in.block_forced && !in.block_every_form &&
+                             in.structures < (in.block_kg == 3 ? 2 : 1) * in.units;
     const bool scratch_rows = in.weighted != 0 || in.radial_basis == 1;
-    c.block = in.block_waves > 0 && (in.average != 2 || outer_rows || outer_lds) && !padded && in.row_bound < kSlotCodeRows &&
+    c.block = in.block_waves > 0 && (in.average != 2 || outer_rows || outer_lds) && !padded && !underfilled && in.row_bound < kSlotCodeRows &&
               !(saving == kLeast && scratch_rows && in.use_mfma && !in.block_forced);
     // By row the radial functions come a species at a time, padded to tiles of
     // 16 rows; the 16x16 kernel forms those of 32 rows at once.  It is the

@@ -87,6 +87,8 @@ def test_one_mode_within_its_limits(rule):
     ((3, 8, 7), "outer", 600, 20, "rows in LDS"), ((5, 2, 6), "off", 600, 20, "tile kernel"),
     ((5, 2, 6), "off", 600, 70, "rows"), ((4, 9, 4), "outer", 600, 20, "tile kernel"),
     ((2, 13, 4), "off", 600, 20, "tile kernel"), ((9, 4, 4), "off", 600, 20, "tile kernel"),
+    # rows in LDS of too few structures, whose centre rows do not fit either
+    ((2, 12, 7), "outer", 150, 50, "tile kernel"), ((2, 12, 7), "outer", 600, 50, "rows in LDS"),
 ])
 def test_modes(rule, shape, average, structures, atoms, expected):
     plan = run_choice.plan_values(*shape, average)
