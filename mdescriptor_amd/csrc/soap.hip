@@ -28,8 +28,6 @@
 
 namespace mdx {
 
-constexpr int kFoldItems = 16;  // rows per split, at least
-constexpr int kFoldSplits = 32; // splits per structure, at most
 
 namespace {
 

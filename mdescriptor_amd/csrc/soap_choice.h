@@ -13,6 +13,9 @@
 namespace mdx {
 
 constexpr int kItemCentres = 32; // centres of an averaged structure per run, at most
+// folded partial rows (k_fold_partials)
+constexpr int kFoldItems = 16;  // rows per split, at least
+constexpr int kFoldSplits = 32; // splits per structure, at most
 // rows of a centre that the 4x4 kernels' slot codes can hold
 constexpr int64_t kSlotCodeRows = int64_t(1) << 27;
 // largest row (features x 8 bytes) the register-coefficient kernel's outer
@@ -68,6 +71,35 @@ inline int64_t run_centres(const ChoiceInput& in, size_t width) {
     };
     while (length < kItemCentres && bytes(length) > static_cast<double>(in.budget)) length *= 2;
     return std::min<int64_t>(length, kItemCentres);
+}
+
+// The same on the tile kernels, whose finalize walks a structure's rows one
+// after another: up to 2 kFoldItems as they are, else their folded splits
+// (k_fold_partials).  A centre of a workgroup's run costs 25-51 us there and a
+// row of the walk 11-23 (four species n 4 l 10 to three n 9 l 10 mu1nu1): the
+// length whose rounds of workgroups and walk are the shortest by a tenth (more
+// rows are also more traffic).  waves: of a workgroup, 8 at a time on a
+// compute unit.  One structure, expansion + finalize in us, runs of 32, runs
+// as short as run_centres takes them, these: three species n 8 l 10 of 1,000
+// atoms 786 + 483, 135 + 529, 207 + 153, of 6,000 820 + 212, 638 + 520, 808 +
+// 212; four n 4 l 10 of 12,000 901 + 252, 1,043 + 334, 897 + 248.
+inline int64_t tile_run_centres(const ChoiceInput& in, size_t width, int waves) {
+    const int64_t slots = in.units * std::max(1, 8 / std::max(1, waves));
+    int64_t best = kItemCentres;
+    double least = 0.0;
+    for (int64_t length = kItemCentres; length >= 1; length /= 2) {
+        const int64_t items = (in.atoms + length - 1) / length + in.structures - 1;
+        const double bytes = static_cast<double>(items + 32 * in.structures) * static_cast<double>(width) * sizeof(double);
+        if (length < kItemCentres && bytes > static_cast<double>(in.budget)) break;
+        const int64_t rows = std::max<int64_t>(1, items / in.structures);
+        const int64_t walk = rows <= 2 * kFoldItems ? rows : std::min<int64_t>((rows + kFoldItems - 1) / kFoldItems, kFoldSplits);
+        const double cost = static_cast<double>((items + slots - 1) / slots * length) + 0.6 * static_cast<double>(walk);
+        if (length == kItemCentres || cost < 0.9 * least) {
+            best = length;
+            least = cost;
+        }
+    }
+    return best;
 }
 
 // The kernel and the decomposition of a run.
@@ -195,7 +227,10 @@ inline Choice choose(const ChoiceInput& in, int saving) {
                       : c.quad          ? in.quad_width
                                         : in.tile_width;
     if (in.average != 0 && c.partials() && !c.block_outer) {
-        c.run = std::min<int64_t>(slice_centres, saving == kFastest ? run_centres(in, c.partial_width) : kItemCentres);
+        const int64_t run = saving != kFastest ? kItemCentres
+                            : c.block          ? run_centres(in, c.partial_width)
+                            : tile_run_centres(in, c.partial_width, c.quad ? in.quad_waves : in.use_mfma ? in.tiles : 4);
+        c.run = std::min<int64_t>(slice_centres, run);
     }
     return c;
 }

@@ -93,3 +93,18 @@ def test_one_mode_within_its_limits(rule):
 def test_modes(rule, shape, average, structures, atoms, expected):
     plan = run_choice.plan_values(*shape, average)
     assert run_choice.mode(rule, plan, run_choice.batch_values(_molecules(structures, atoms), 4.0)) == expected
+
+
+@pytest.mark.parametrize("atoms,waves,longest,shortest", [
+    (1000, 8, 8, 4), (3000, 8, 16, 16), (6000, 8, 32, 32), (6000, 4, 16, 16), (12000, 4, 32, 32), (40000, 16, 32, 32),
+])
+def test_runs_of_a_structure_on_the_tile_kernels(rule, atoms, waves, longest, shortest):
+    """One structure's centres in runs: short ones fill the device, but the
+    finalize walks their rows one after another."""
+
+    plan = run_choice.plan_values(3, 8, 10, "inner")
+    plan["quad_waves"] = waves
+    cell = dict(structures=1, atoms=atoms, largest_structure=atoms, most_images=27 * atoms, row_bound=512, units=256,
+                budget=1 << 30)
+    c = run_choice.evaluate(rule, {**plan, **cell})
+    assert c["quad"] and shortest <= c["run"] <= longest
