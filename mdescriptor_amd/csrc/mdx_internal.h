@@ -513,9 +513,8 @@ struct mdx_soap_plan {
     // not used), radial groups, MFMA instructions per step, lane constants
     int quad_waves = 0, quad_kg = 0, quad_instr = 0;
     mdx::DeviceBuffer d_quad_lanes;
-    // register-coefficient kernel (soap_block.hip), default options and
-    // average "off" only: wavefronts (0: not used), radial groups,
-    // coefficient registers, lane tables
+    // register-coefficient kernel (soap_block.hip): wavefronts (0: no compiled
+    // shape holds the plan), radial groups, coefficient registers, lane tables
     int block_waves = 0, block_kg = 0, block_ncr = 0;
     bool block_float32 = false; // float32 exps (block_float32_exps)
     bool block_every_form = false; // BlockShape::every_form

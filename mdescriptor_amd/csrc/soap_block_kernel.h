@@ -1,7 +1,8 @@
-// Kernels 2-4 for the default SOAP options (GTO basis, no weighting, no
-// compression) with the coefficients held in registers: neighbour expansion
-// on 4x4x4 FP64 matrix-core blocks, beta fold, power spectrum on 16x16x4 FP64
-// Gram tiles and the row write (soap.cpp:864-930, 997-1013).
+// Kernels 2-4 with the coefficients held in registers: neighbour expansion on
+// 4x4x4 FP64 matrix-core blocks, beta fold, power spectrum on 16x16x4 FP64
+// Gram tiles and the row write (soap.cpp:864-930, 948-1013), for l_max 2-9 and
+// up to twelve radial channels, both radial bases, every weighting,
+// compression and average (soap_block.h: modes and forms).
 //
 // One workgroup of T wavefronts handles one centre at a time.  Degree l is
 // owned by one wavefront, which keeps everything of that degree in its

