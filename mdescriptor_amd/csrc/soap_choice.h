@@ -84,16 +84,22 @@ inline int64_t run_centres(const ChoiceInput& in, size_t width) {
 // atoms 786 + 483, 135 + 529, 207 + 153, of 6,000 820 + 212, 638 + 520, 808 +
 // 212; four n 4 l 10 of 12,000 901 + 252, 1,043 + 334, 897 + 248.
 inline int64_t tile_run_centres(const ChoiceInput& in, size_t width, int waves) {
+    // (as many structures as compute units: splitting them adds rows, 3,000
+    // molecules of 2-8 atoms mu2 l 0 40 us whole and 47 in fours)
+    if (in.structures >= in.units) return kItemCentres;
     const int64_t slots = in.units * std::max(1, 8 / std::max(1, waves));
     int64_t best = kItemCentres;
     double least = 0.0;
     for (int64_t length = kItemCentres; length >= 1; length /= 2) {
-        const int64_t items = (in.atoms + length - 1) / length + in.structures - 1;
+        // (no run is longer than the largest structure)
+        const int64_t centres = std::min(length, in.largest_structure);
+        const int64_t items =
+            length >= in.largest_structure ? in.structures : (in.atoms + in.structures * (length - 1)) / length;
         const double bytes = static_cast<double>(items + 32 * in.structures) * static_cast<double>(width) * sizeof(double);
         if (length < kItemCentres && bytes > static_cast<double>(in.budget)) break;
         const int64_t rows = std::max<int64_t>(1, items / in.structures);
         const int64_t walk = rows <= 2 * kFoldItems ? rows : std::min<int64_t>((rows + kFoldItems - 1) / kFoldItems, kFoldSplits);
-        const double cost = static_cast<double>((items + slots - 1) / slots * length) + 0.6 * static_cast<double>(walk);
+        const double cost = static_cast<double>((items + slots - 1) / slots * centres) + 0.6 * static_cast<double>(walk);
         if (length == kItemCentres || cost < 0.9 * least) {
             best = length;
             least = cost;

@@ -95,6 +95,15 @@ def test_modes(rule, shape, average, structures, atoms, expected):
     assert run_choice.mode(rule, plan, run_choice.batch_values(_molecules(structures, atoms), 4.0)) == expected
 
 
+def test_small_structures_are_not_split(rule):
+    """Molecules of at most a run: one row each, nothing for the finalize to add."""
+
+    plan = run_choice.plan_values(1, 3, 0, "inner", options={"compression": "mu2"})
+    molecules = dict(structures=3000, atoms=15000, largest_structure=8, most_images=8, row_bound=16, units=256,
+                     budget=50 << 20)
+    assert run_choice.evaluate(rule, {**plan, **molecules})["run"] >= 8
+
+
 @pytest.mark.parametrize("atoms,waves,longest,shortest", [
     (1000, 8, 8, 4), (3000, 8, 16, 16), (6000, 8, 32, 32), (6000, 4, 16, 16), (12000, 4, 32, 32), (40000, 16, 32, 32),
 ])
