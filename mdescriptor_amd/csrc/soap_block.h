@@ -23,17 +23,21 @@ namespace mdx {
 //   outer LDS    outer averages, a workgroup per structure: every centre's
 //                power spectrum added into the structure's float64 row in
 //                LDS and the mean written once
+//   inner runs   the first of the two launches above by itself (shapes compiled
+//                in every form: with a row's end in the same kernel 500
+//                structures of 70-100 atoms, four species n 5 l 6, took 457 us
+//                instead of 403)
 // Each takes neighbour weights (row_w) and every compression: mu1nu1
 // (summed: each channel against the species-summed channels) as a branch at
 // the end of a row, the others through the plan's tables.
-constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuterLds = 3;
+constexpr int kBlockRows = 0, kBlockInner = 1, kBlockInnerSmall = 2, kBlockOuterLds = 3, kBlockInnerRuns = 4;
 // ... and forms: unweighted, weighted (the weights may be 1), the polynomial
 // basis (weighted the same way): the radial functions come from memory
 // (launch_poly_radial) instead of exps, rows and inner averages only, up to
 // two radial groups (its normalisation fails past eight channels);
-// unweighted float32 rows of float64 tables; and weighted rows of the tables'
-// own type (shapes compiled in every form).
-constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2, kBlockHalf = 3, kBlockWeightedRows = 4;
+// unweighted float32 rows of float64 tables; and weighted rows and inner
+// averages of the tables' own type (shapes compiled in every form).
+constexpr int kBlockPlain = 0, kBlockWeighted = 1, kBlockPolynomial = 2, kBlockHalf = 3, kBlockWeightedFull = 4;
 constexpr int kBlockPolyGroups = 2;
 
 // Launch arguments (one struct, passed by value).

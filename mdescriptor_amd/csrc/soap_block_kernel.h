@@ -704,7 +704,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
     // choice per store cost float64 rows 1-2 %, weighted ones 4-6 %: 1,000
     // molecules of five species n 8 l 8, crossover, 366 and 401 us)
     const bool half_rows =
-        ES == 8 && (FORM == kBlockHalf || (kWeighted && FORM != kBlockWeightedRows && a.out_bytes == 4));
+        ES == 8 && (FORM == kBlockHalf || (kWeighted && FORM != kBlockWeightedFull && a.out_bytes == 4));
     // row end: C <- (S_lm C)^T beta^T scaled by scale0, the power spectrum of
     // the owned degrees to output row row0, and C back to zero
     auto row_end = [&](int64_t row0, double scale0) {
@@ -1028,7 +1028,7 @@ __device__ __forceinline__ void block_role(const BlockArgs& a, double* lds, cons
                     }
                 }
                 __syncthreads();
-            } else if (MODE == kBlockInner && a.partial_out != nullptr) {
+            } else if (MODE == kBlockInnerRuns || (MODE == kBlockInner && a.partial_out != nullptr)) {
                 // the run's summed coefficient registers to its partial row
                 double* part = a.partial_out + row0 * kPartWidth + kPartBase + lane;
                 unroll<NU>([&](auto uc) {
@@ -1189,12 +1189,13 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
     using Rows = std::integral_constant<int, kBlockRows>;
     using Inner = std::integral_constant<int, kBlockInner>;
     using Small = std::integral_constant<int, kBlockInnerSmall>;
+    using Runs = std::integral_constant<int, kBlockInnerRuns>;
     using Outer = std::integral_constant<int, kBlockOuterLds>;
     using Plain = std::integral_constant<int, kBlockPlain>;
     using Weighted = std::integral_constant<int, kBlockWeighted>;
     using Polynomial = std::integral_constant<int, kBlockPolynomial>;
     using Half = std::integral_constant<int, kBlockHalf>;
-    using WeightedRows = std::integral_constant<int, kBlockWeightedRows>;
+    using WeightedFull = std::integral_constant<int, kBlockWeightedFull>;
     if (a.polynomial != 0) {
         if constexpr (KG <= kBlockPolyGroups) {
             if (a.struct_offsets == nullptr) launch(F64{}, Rows{}, Polynomial{}); else launch(F64{}, Inner{}, Polynomial{});
@@ -1207,28 +1208,24 @@ void launch_shape(hipStream_t stream, const BlockArgs& a, int64_t count) {
         // (rows of the (3, 1, 1) shape 76.4 -> 80.0 us, of (9, 3, 1) 1,829 -> 1,866 us)
         auto typed = [&](auto m) {
             if (f32) {
-                if (weighted) launch(F32{}, m, Weighted{}); else launch(F32{}, m, Plain{});
+                if (weighted) launch(F32{}, m, WeightedFull{}); else launch(F32{}, m, Plain{});
+            } else if (a.out_bytes == 4) {
+                launch(F64{}, m, Weighted{});
             } else {
-                if (weighted || a.out_bytes == 4) launch(F64{}, m, Weighted{}); else launch(F64{}, m, Plain{});
+                if (weighted) launch(F64{}, m, WeightedFull{}); else launch(F64{}, m, Plain{});
             }
         };
         if (outer) {
             if (weighted) launch(F64{}, Outer{}, Weighted{}); else launch(F64{}, Outer{}, Plain{});
         } else if (a.struct_offsets == nullptr) {
-            if (weighted && a.out_bytes == a.table_dtype) {
-                if (f32) launch(F32{}, Rows{}, WeightedRows{}); else launch(F64{}, Rows{}, WeightedRows{});
-            } else if (f32) {
-                launch(F32{}, Rows{}, Plain{});
-            } else if (weighted || a.out_bytes == 4) {
-                launch(F64{}, Rows{}, Weighted{});
-            } else {
-                launch(F64{}, Rows{}, Plain{});
-            }
+            typed(Rows{});
         } else if (a.small_structures) {
             // (weighted: float64 exps)
             if (f32) launch(F32{}, Small{}, Plain{});
             else if (weighted || a.out_bytes == 4) launch(F64{}, Small{}, Weighted{});
             else launch(F64{}, Small{}, Plain{});
+        } else if (a.partial_out != nullptr) {
+            typed(Runs{});
         } else {
             typed(Inner{});
         }
