@@ -410,6 +410,7 @@ Fold fold_of(int64_t most_items) {
 }
 
 static_assert(kSlotCodeRows == kQuadMaxRows, "one limit for both 4x4 kernels");
+static_assert(kFirstSlots == kMinSlotCap, "the slots of a first search");
 ChoiceInput choice_input(const mdx_soap_plan& p, const PreparedBatch& pb, const DeviceGraph& g) {
     ChoiceInput in;
     in.average = p.average;

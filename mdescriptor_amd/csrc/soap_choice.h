@@ -18,6 +18,7 @@ constexpr int kFoldItems = 16;  // rows per split, at least
 constexpr int kFoldSplits = 32; // splits per structure, at most
 // rows of a centre that the 4x4 kernels' slot codes can hold
 constexpr int64_t kSlotCodeRows = int64_t(1) << 27;
+constexpr int64_t kFirstSlots = 512; // rows a centre's slots hold at first (kMinSlotCap)
 // largest row (features x 8 bytes) the register-coefficient kernel's outer
 // averages accumulate in LDS
 constexpr int64_t kBlockOuterLdsBytes = 48 * 1024;
@@ -59,11 +60,22 @@ struct ChoiceInput {
     int64_t budget = 0;   // bytes its partial rows may take
 };
 
+// Rows a centre the rule counts with: the first slots' width while the rows
+// have not been counted, and after (both entry points then decide alike).
+inline int64_t planned_rows(const ChoiceInput& in) {
+    return std::max(in.row_bound, std::min(kFirstSlots, (in.most_images + 15) / 16 * 16));
+}
+
 // Centres per run of an averaged structure: kItemCentres where the batch then
 // still has a few runs for every compute unit, shorter for smaller batches
 // (8,192 atoms at 32 are 256 runs, one workgroup a compute unit) as far as
 // their partial rows (width doubles each, and the folded ones) fit the budget.
+// About three runs of kItemCentres a compute unit are enough: more of them only
+// add rows (200 structures of 100-160 atoms, four species n 8 l 6, 388 us with
+// runs of 32, 409 with runs of 12; 500 of 70-100 419 and 472; 60 of 100-160,
+// 300 runs of 32, 250 and 183 with runs of 3).
 inline int64_t run_centres(const ChoiceInput& in, size_t width) {
+    if ((in.atoms + in.structures * (kItemCentres / 2)) / kItemCentres >= 3 * in.units) return kItemCentres;
     const int64_t fill = 8 * in.units;
     int64_t length = std::max<int64_t>(1, std::min<int64_t>(kItemCentres, in.atoms / fill));
     auto bytes = [&](int64_t len) {
@@ -196,20 +208,20 @@ inline Choice choose(const ChoiceInput& in, int saving) {
     // and 922; 2,000 molecules of 9-29 atoms of two, three, six species 753 and
     // 958, 1,313 and 1,067, 1,709 and 1,384; l 2 n 6, 4,000 atoms of nine 1,276
     // and 1,024.
-    const bool short_tiles = in.S > 6 || (in.S > 2 && std::min(in.most_images, in.row_bound) < 32 * in.S);
+    const bool short_tiles = in.S > 6 || (in.S > 2 && std::min(in.most_images, planned_rows(in)) < 32 * in.S);
     c.poly_inside = in.radial_basis == 1 && !c.block && (saving == kLeast || (in.L <= 8 && in.n <= 8 && short_tiles));
     const size_t block_width = c.block ? in.block_width : 0;
     // A few small periodic structures hold thousands of pairs each (a
     // workgroup takes about a microsecond per 32 of them): runs too.
     const bool spread = saving == kFastest && !in.block_forced && in.structures < in.units &&
-                        in.largest_structure * std::min(in.most_images, in.row_bound) > kBlockSpreadPairs &&
+                        in.largest_structure * std::min(in.most_images, planned_rows(in)) > kBlockSpreadPairs &&
                         static_cast<double>(in.atoms + 5 * in.structures) * static_cast<double>(block_width) * 8.0 <=
                             static_cast<double>(in.budget);
     // Centres of the polynomial basis that a slice of radial functions holds.
     // A structure formed in one workgroup needs all of its centres at once: one
     // past that (12,000 atoms among 1,024 molecules: 1.2 GB at l 2) sums runs,
     // and no run is longer.
-    const PolyLayout poly = poly_layout(in.row_bound, in.S, in.L, in.n, c.block);
+    const PolyLayout poly = poly_layout(planned_rows(in), in.S, in.L, in.n, c.block);
     const int64_t slice_centres =
         in.radial_basis != 1 || c.poly_inside
             ? std::numeric_limits<int64_t>::max()
@@ -236,7 +248,14 @@ inline Choice choose(const ChoiceInput& in, int saving) {
         const int64_t run = saving != kFastest ? kItemCentres
                             : c.block          ? run_centres(in, c.partial_width)
                             : tile_run_centres(in, c.partial_width, c.quad ? in.quad_waves : in.use_mfma ? in.tiles : 4);
-        c.run = std::min<int64_t>(slice_centres, run);
+        // by row, a slice of radial functions holds enough runs to fill the
+        // device (kPolyLeastWaves; 500 structures of 70-100 atoms, n 8 l 1 of
+        // three species, three slices of 585 runs of one wavefront each:
+        // 7.6 ms, in the kernel itself 5.8)
+        const int64_t fill = c.block || saving != kFastest || slice_centres >= in.atoms
+                                 ? slice_centres
+                                 : std::max<int64_t>(1, slice_centres * in.tiles / kPolyLeastWaves);
+        c.run = std::min<int64_t>(fill, run);
     }
     return c;
 }

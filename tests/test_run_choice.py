@@ -117,3 +117,24 @@ def test_runs_of_a_structure_on_the_tile_kernels(rule, atoms, waves, longest, sh
                 budget=1 << 30)
     c = run_choice.evaluate(rule, {**plan, **cell})
     assert c["quad"] and shortest <= c["run"] <= longest
+
+
+def test_runs_that_already_fill_the_device_stay_long(rule):
+    plan = run_choice.plan_values(4, 8, 6, "inner")
+    for structures, atoms, run in ((500, 85, 32), (200, 130, 32), (60, 130, 3)):
+        batch = dict(structures=structures, atoms=structures * atoms, largest_structure=atoms + 30,
+                     most_images=atoms + 30, row_bound=160, units=256, budget=1 << 30)
+        c = run_choice.evaluate(rule, {**plan, **batch})
+        assert c["block_runs"] and c["run"] == run
+
+
+def test_slices_of_radial_rows_hold_runs_for_the_device(rule):
+    """By row: runs short enough that a slice has 2,048 wavefronts of them."""
+
+    plan = run_choice.plan_values(3, 8, 1, "inner", options={"polynomial": True})
+    batch = dict(structures=500, atoms=42500, largest_structure=100, most_images=100, row_bound=112, units=256,
+                 budget=1 << 30)
+    c = run_choice.evaluate(rule, {**plan, **batch})
+    assert c["poly_centre"] and not c["block"]
+    slice_centres = SLICE // (8 * c["poly_centre"])
+    assert slice_centres // c["run"] >= 2048
