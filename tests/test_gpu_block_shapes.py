@@ -353,3 +353,24 @@ def test_molecules_of_padded_shapes(hip_context, oracle, shape, average, compres
             assert scaled_error(values, oracle.soap(batch, **arguments)) <= GATES["float64"]
     finally:
         plan.close()
+
+
+def test_runs_keep_the_rows_sums(hip_context, oracle):
+    """Inner averages from many short runs: their rows are summed before the
+    beta fold, which amplifies the sums' rounding, so the error stays near that
+    of the oracle's own order of sums (1e-13 of the row; the gate is 1e-10)."""
+
+    rng = np.random.default_rng(8)
+    sizes = (400, 380)
+    batch = _structures(8, sizes, SPECIES[:2])
+    batch.positions = batch.positions + rng.uniform(-0.1, 0.1, batch.positions.shape)
+    alphas, betas = basis_gto(4.0, 8, 3)
+    arguments = dict(species=SPECIES[:2], n_max=8, l_max=3, r_cut=4.0, sigma=1.0, alphas=alphas, betas=betas,
+                     average="inner")
+    plan = _hip.SoapPlan(hip_context, dtype="float64", **arguments)
+    try:
+        values, timing = plan.compute(batch)
+    finally:
+        plan.close()
+    assert timing["expansion_tiles"] <= -1000
+    assert scaled_error(values, oracle.soap(batch, **arguments)) <= 1e-11
